@@ -1,0 +1,84 @@
+"""GPU parity of the prefill-chunk attention (more than 8 tokens: scores with a position per lane,
+softmax in place, P.V with a dim per lane) against the step kernels over the same tokens in passes
+of at most 8, which test_gpu_attn.py and the end-to-end tests pin.
+
+Bar: bit-exact for the output, its A8 and both caches (every sum is the same ordered chain). Cases
+at the tiles' edges: 9 rows, ragged row groups (3 heads per KV group), 64-position tiles entered and
+left inside the chunk, softmax segments of 4096, caches past 8192 positions, head sizes 64 to 512."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from nibblemac_amd.nmx import A8, AttnArgs
+from tests.test_gpu_attn import cache_bytes
+from tests.test_gpu_q4k import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def passes(dev, host, shape, step):
+    """The chunk in passes of `step` tokens: o [n][nh hd], its A8 (codes, d, fsum per block and
+    token), the caches."""
+    n, nh, nkv, hd, max_ctx, kvt, pos0 = shape
+    kc, vc = dev.to_device(host["kc"]), dev.to_device(host["vc"])
+    const = {k: dev.to_device(host[k]) for k in ("q_norm", "k_norm", "cos", "sin")}
+    nb, outs = nh * hd // 32, []
+    for t0 in range(0, n, step):
+        m = min(step, n - t0)
+        q, k, v = (dev.to_device(host[x][t0:t0 + m]) for x in ("q", "k_in", "v_in"))
+        pos = dev.to_device(np.array([pos0 + 3], np.int32))
+        o = dev.zeros((m, nh * hd), np.float32)
+        a8 = (dev.zeros((nb, m, 32), np.int8), dev.zeros((nb, m), np.float32),
+              dev.zeros((nb, m), np.float32))
+        sc = dev.zeros((m, nh, max_ctx), np.float32)
+        a = AttnArgs(m, nh, nkv, hd, hd // 4, max_ctx, q.ptr, k.ptr, v.ptr, const["q_norm"].ptr,
+                     const["k_norm"].ptr, 1e-6, np.float32(1.0 / np.sqrt(hd)), const["cos"].ptr,
+                     const["sin"].ptr, kc.ptr, vc.ptr, pos.ptr, t0 - 3, o.ptr,
+                     A8(*[b.ptr for b in a8]), sc.ptr, kvt)
+        dev.attn_prep(a)
+        dev.attn(a)
+        dev.sync()
+        outs.append((o.numpy(), *[b.numpy() for b in a8]))
+        for b in (q, k, v, pos, o, *a8, sc):
+            b.free()
+    return dict(o=np.concatenate([x[0] for x in outs]),
+                **{k: np.concatenate([x[i] for x in outs], axis=1)
+                   for i, k in ((1, "aq"), (2, "ad"), (3, "afs"))},
+                kc=kc.numpy(), vc=vc.numpy())
+
+
+CASES = [
+    # n, query heads, KV heads, head size, max_ctx, kv dtype, position of token 0
+    (9, 8, 2, 256, 1024, 0, 0),
+    (64, 8, 2, 256, 1024, 0, 448),
+    (64, 8, 2, 256, 1000, 0, 936),     # the last positions of a ragged cache
+    (33, 8, 2, 256, 1024, 1, 40),
+    (64, 8, 2, 256, 1024, 2, 63),
+    (17, 6, 2, 128, 512, 0, 50),       # three heads per group: rows of a wave straddle tokens
+    (12, 4, 4, 64, 256, 0, 10),
+    (20, 8, 1, 512, 512, 1, 100),
+    (40, 4, 2, 64, 8192, 0, 4080),     # rows across the first softmax segment's end
+    (10, 2, 1, 64, 16384, 2, 9000),    # past the in-LDS step kernel, three segments
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "n%d_h%d_%d_hd%d_ctx%d_kv%d_pos%d" % c)
+def test_chunk_equals_steps(dev, case):
+    n, nh, nkv, hd, max_ctx, kvt, pos0 = case
+    print(f"[case] attn chunk {case}", flush=True)
+    rng = np.random.default_rng(n + 7 * hd + pos0)
+    ang = rng.uniform(0, 2 * np.pi, (max_ctx, hd // 8))
+    host = dict(
+        q=rng.standard_normal((n, nh, 2 * hd)).astype(np.float32),
+        k_in=rng.standard_normal((n, nkv * hd)).astype(np.float32),
+        v_in=rng.standard_normal((n, nkv * hd)).astype(np.float32),
+        q_norm=rng.uniform(0.5, 1.5, hd).astype(np.float32),
+        k_norm=rng.uniform(0.5, 1.5, hd).astype(np.float32),
+        cos=np.cos(ang).astype(np.float32), sin=np.sin(ang).astype(np.float32),
+        kc=cache_bytes(rng, kvt, nkv, max_ctx, hd), vc=cache_bytes(rng, kvt, nkv, max_ctx, hd),
+    )
+    want = passes(dev, host, case, 8)
+    got = passes(dev, host, case, 64)
+    for k in want:
+        assert_bits_equal(got[k], want[k], k)
