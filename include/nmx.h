@@ -305,7 +305,8 @@ int nmx_lin_post(nmx_ctx *ctx, const float *o, int o_stride, const float *z, int
  * its A8), with identical results; the conv outputs, gates and o stay on chip. pre.out,
  * pre.beta, pre.decay, rule.qkv, rule.decay, rule.beta and rule.o are only used (and then
  * must be valid buffers) when the shape is outside the fused kernel's limits and the three
- * kernels run instead. */
+ * kernels run instead, and by the chunk kernels that take more than 8 tokens without a log
+ * when all of them are given and overlap no other argument. */
 typedef struct {
     nmx_lin_pre_args pre;
     nmx_lin_args rule;

@@ -23,6 +23,7 @@
  * instruction, and issuing them took about 2 us per workgroup in the mixer).
  * Log rows keep the reference layout [n][heads][dk + dv + 1] = k | delta | decay. */
 #include "nmx_internal.h"
+#include "nmx_linc.h"
 #include "nmx_a8.h"
 
 namespace {
@@ -250,6 +251,7 @@ int nmx_lin_rule(nmx_ctx *ctx, const nmx_lin_args *a) {
     if (!ctx) return -1;
     if (validate(ctx, a, "nmx_lin_rule")) return -1;
     if (a->n < 1) return nmx_fail(ctx, "nmx_lin_rule: n=%d (>= 1 needed)", a->n);
+    if (nmx_lin_rulec_ok(*a)) return nmx_lin_rulec(ctx, *a);
     return dispatch(ctx, *a);
 }
 

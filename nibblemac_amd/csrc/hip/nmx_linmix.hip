@@ -13,6 +13,7 @@
  * of nmx_lin_rule (lane c of the quad holds keys [c dk/4, (c+1) dk/4) of its column in VGPRs);
  * the conv stage has one thread per channel; the norms run as 4-lane ordered chains. */
 #include "nmx_internal.h"
+#include "nmx_linc.h"
 #include "nmx_math.h"
 #include "nmx_a8.h"
 
@@ -441,6 +442,48 @@ int launch_mix(nmx_ctx *ctx, const LinMix &m, size_t lds) {
     return 0;
 }
 
+/* Whether the chunk kernels (nmx_linc.hip) take the mixer: more than 8 tokens without a log, and
+ * intermediate buffers that pass between the kernels (the fused kernel does without them, so a
+ * caller may have left them out) and overlap nothing that a later kernel reads or writes. 64
+ * tokens, 16 heads of 128: 5.6 + 39.8 + 4.8 us against 97-100 us for lin_mix_k, whose time per token
+ * is 1.45 us above about 5 us of setup. */
+bool chunk_ok(const nmx_lin_mix_args &a) {
+    const nmx_lin_pre_args &p = a.pre;
+    const nmx_lin_args &r = a.rule;
+    if (!nmx_lin_rulec_ok(r) || p.conv_k != 4 || p.xin || p.dk > 256 || p.C % 32 || r.heads < 1 ||
+        r.heads > 256 || r.rep < 1 || r.heads % r.rep || r.dv < 32 || r.dv > 512 || r.keep < 0 ||
+        r.keep > 64 || (r.keep > 0 && !r.pend) || p.n * p.heads > 4096 || !p.raw || !p.state ||
+        !p.conv_w || !p.b_in || !p.a_in || !p.dt_bias || (!p.A_log && !p.A) || !p.out || !p.beta ||
+        !p.decay || !r.S || !r.o || p.raw_stride < p.C || p.g_stride < p.heads)
+        return false;
+    if (r.qkv != p.out || r.qkv_stride != p.C || r.decay != p.decay || r.beta != p.beta ||
+        r.o_stride < r.heads * r.dv)
+        return false;
+    const size_t n = (size_t)p.n, C = (size_t)p.C, g = n * p.heads * 4, vd = (size_t)r.heads * r.dv;
+    struct Span {
+        const void *p;
+        size_t b;
+    };
+    const Span w[] = {{p.out, n * C * 4}, {p.beta, g}, {p.decay, g},
+             {r.o, ((n - 1) * r.o_stride + vd) * 4}, {r.S, vd * r.dk * 4}, {p.state, 3 * C * 4}},
+      other[] = {{p.raw, ((n - 1) * p.raw_stride + C) * 4}, {p.conv_w, C * 16},
+                 {p.b_in, ((n - 1) * p.g_stride + p.heads) * 4},
+                 {p.a_in, ((n - 1) * p.g_stride + p.heads) * 4},
+                 {p.A, p.A ? (size_t)p.heads * 4 : 0}, {p.A_log, p.A_log ? (size_t)p.heads * 4 : 0},
+                 {p.dt_bias, (size_t)p.heads * 4},
+                 {r.pend, (size_t)r.keep * r.heads * (r.dk + r.dv + 1) * 4},
+                 {a.z, ((n - 1) * a.z_stride + vd) * 4}, {a.norm_w, (size_t)r.dv * 4},
+                 {a.y, a.y ? ((n - 1) * a.y_stride + vd) * 4 : 0}, {a.a8.q, a.a8.q ? n * vd : 0},
+                 {a.a8.d, a.a8.q ? n * vd / 8 : 0}, {a.a8.fs, a.a8.q ? n * vd / 8 : 0}};
+    for (size_t i = 0; i < sizeof w / sizeof *w; i++) {
+        for (size_t k = i + 1; k < sizeof w / sizeof *w; k++)
+            if (nmx_overlap(w[i].p, w[i].b, w[k].p, w[k].b)) return false;
+        for (const Span &x : other)
+            if (nmx_overlap(w[i].p, w[i].b, x.p, x.b)) return false;
+    }
+    return true;
+}
+
 } // namespace
 
 extern "C" {
@@ -468,6 +511,11 @@ int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) {
     const bool fused = r.rep == 1 && (dk == 64 || dk == 128) && 4 * dv <= MIX_MAX_THREADS &&
                        dk <= dv && 2 * dk + dv <= 4 * dv - 64 && lds <= MIX_LDS && vec_ok &&
                        !(r.log0 && !r.log);
+    if (chunk_ok(*a)) { /* the chunk kernels, through the structs' intermediate buffers */
+        if (nmx_lin_mixc(ctx, p, r)) return -1;
+        return nmx_lin_post(ctx, r.o, r.o_stride, a->z, a->z_stride, a->norm_w, n, r.heads, dv,
+                            a->eps, a->y, a->y_stride, a->a8);
+    }
     if (!fused) { /* the separate kernels, through the intermediate buffers of the structs */
         if (nmx_lin_pre(ctx, &p) || nmx_lin_rule(ctx, &r)) return -1;
         return nmx_lin_post(ctx, r.o, r.o_stride, a->z, a->z_stride, a->norm_w, n, r.heads, dv,

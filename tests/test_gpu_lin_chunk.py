@@ -1,0 +1,84 @@
+"""GPU parity of the DeltaNet chunk kernels (more than 8 tokens, no log: conv, norms and gates with
+the tokens in parallel, then kv chains and skewed o chains in waves of their own).
+
+The recurrence is compared with the oracle and the whole mixer with lin_mix_k, the one-launch kernel
+that takes the same pass when the intermediate buffers are left out. Bar: bit-exact for outputs,
+recurrent state and conv state. Sizes at the pipeline's edges: 9 tokens (less than the 15 steps a
+sum takes), 16 and 17 (one batch, one more token), 48, 63, 64 (the ring of 4 batches wraps), pending
+replays, shared key heads, dk 64 to 256, a last column group that is not 16 wide."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from nibblemac_amd.nmx import A8, LinArgs, LinMixArgs, LinPreArgs
+from tests.refmath import state_from_dev, state_to_dev
+from tests.test_gpu_linmix import make_case, p, run
+from tests.test_gpu_q4k import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("case", [
+    # n, heads, rep, dk, dv, keep
+    (9, 2, 1, 128, 128, 0), (16, 2, 1, 128, 128, 3), (17, 4, 2, 128, 64, 0), (48, 2, 1, 64, 64, 9),
+    (63, 2, 1, 256, 32, 1), (64, 16, 1, 128, 128, 0), (64, 3, 3, 64, 24, 0), (31, 2, 1, 128, 8, 5),
+], ids=lambda c: "n%d_h%d_rep%d_dk%d_dv%d_keep%d" % c)
+def test_rule_equals_oracle(dev, case):
+    n, heads, rep, dk, dv, keep = case
+    print(f"[case] lin chunk rule {case}", flush=True)
+    rng = np.random.default_rng(n + dk + dv + keep)
+    kd, stride = heads // rep * dk, 2 * (heads // rep) * dk + heads * dv
+    qkv = rng.standard_normal((n, stride)).astype(np.float32)
+    qkv[:, :2 * kd] *= np.float32(dk ** -0.5)
+    decay = rng.uniform(0.8, 1.0, (n, heads)).astype(np.float32)
+    beta = rng.uniform(0.1, 0.9, (n, heads)).astype(np.float32)
+    S = (rng.standard_normal((heads, dk, dv)) * 0.05).astype(np.float32)
+    S.ravel()[::7] = -0.0
+    pend = (rng.standard_normal((max(keep, 1), heads, dk + dv + 1)) * 0.1).astype(np.float32)
+    want_S, want_o, _ = oracle.lin_rule(qkv, decay, beta, S, n=n, heads=heads, rep=rep, dk=dk, dv=dv,
+                                        pend=pend, keep=keep)
+    dS, dq, dd, db = (dev.to_device(x) for x in (state_to_dev(S, heads, dk, dv), qkv, decay, beta))
+    o, dp = dev.zeros((n, heads * dv), np.float32), dev.to_device(pend)
+    dev.lin_rule(n=n, heads=heads, rep=rep, dk=dk, dv=dv, qkv_stride=stride, o_stride=heads * dv,
+                 qkv=dq, decay=dd, beta=db, S=dS, o=o, pend=dp, keep=keep)
+    dev.sync()
+    assert_bits_equal(o.numpy(), want_o, "o")
+    assert_bits_equal(state_from_dev(dS.numpy(), heads, dk, dv), want_S, "state")
+
+
+def one_launch(dev, c):
+    """The pass through lin_mix_k: no intermediate buffers."""
+    n, heads, dk, dv, C = (c[k] for k in ("n", "heads", "dk", "dv", "C"))
+    d = {k: dev.to_device(v) for k, v in c["host"].items()}
+    nb = heads * dv // 32
+    y = dev.zeros((n, heads * dv), np.float32)
+    aq, ad, afs = (dev.zeros((nb, n, 32), np.int8), dev.zeros((nb, n), np.float32),
+                   dev.zeros((nb, n), np.float32))
+    pre = LinPreArgs(n, C, c["K"], dk, c["kd"], p(d["raw"]), C, None, p(d["state"]), p(d["conv_w"]),
+                     None, np.float32(1.0 / np.sqrt(dk)), 1e-6, p(d["b"]), p(d["a"]), heads, heads,
+                     p(d["A_log"]), None, p(d["dt_bias"]), None, None)
+    rule = LinArgs(n, heads, 1, dk, dv, C, heads * dv, None, None, None, p(d["S"]), None, None,
+                   p(d["pend"]), c["keep"], 0, None)
+    dev.lin_mix(LinMixArgs(pre, rule, p(d["z"]), heads * dv, p(d["norm_w"]), 1e-6, p(y), heads * dv,
+                           A8(p(aq), p(ad), p(afs))))
+    dev.sync()
+    return dict(aq=aq.numpy(), ad=ad.numpy(), afs=afs.numpy(), y=y.numpy(), S=d["S"].numpy(),
+                state=d["state"].numpy())
+
+
+@pytest.mark.parametrize("case", [
+    # n, heads, dk, dv, keep
+    (9, 4, 128, 128, 0), (13, 4, 128, 128, 4), (33, 4, 64, 64, 0), (64, 16, 128, 128, 0),
+    (57, 2, 64, 128, 2),
+], ids=lambda c: "n%d_h%d_dk%d_dv%d_keep%d" % c)
+def test_mixer_equals_one_launch(dev, case):
+    n, heads, dk, dv, keep = case
+    print(f"[case] lin chunk mixer {case}", flush=True)
+    rng = np.random.default_rng(3 * n + heads + dk + keep)
+    c = make_case(dev, rng, n, heads, 1, dk, dv, logged=False, keep=keep)
+    want = one_launch(dev, c)
+    got = run(dev, c, fused=True)
+    for k in want:
+        assert_bits_equal(got[k], want[k], k)
