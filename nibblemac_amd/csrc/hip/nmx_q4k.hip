@@ -20,6 +20,7 @@
 #include <mutex>
 
 #include "nmx_internal.h"
+#include "nmx_math.h"
 #include "nmx_a8.h"
 #include "nmx_lanes.h"
 #include "nmx_rms.h"
@@ -777,34 +778,45 @@ __global__ __launch_bounds__(1024) void q4k_mv_ks_k(SegTable tab, int cols, int 
  * v_mfma_i32_16x16x32_i8 per (16 rows, 16 vectors, 32-column block), then the reference's
  * ordered per-block FMA pair on the 16 x 16 result in registers.
  *
- * A wave owns 16 rows (four 4-row tiles) and NT tiles of 16 vectors; a workgroup of WAVES waves
- * shares the activations of its vectors, staged in LDS one superblock at a time; the weights and
- * activations of superblock sb + DIST are loaded into registers while sb is used (DIST = 2 for
- * single-wave workgroups, whose latency nothing else on the CU hides; 1 where VGPRs are
- * short).
+ * A workgroup of MM_S waves owns 16 rows x 16 vectors, its waves the superblocks in turn (wave w
+ * takes w, w + MM_S, ..). Only the FMA chain is serial, 8 of about 40 instructions per block, so a
+ * wave loads its superblock, decodes the scales, forms the dots and (D*s)*d in registers on its own,
+ * and runs its 8 blocks' chains when the accumulators reach it: they pass from wave to wave in LDS
+ * behind a turn counter (a wave waits only for waves with earlier superblocks, so the turns always
+ * come). A chunk has few tiles for the chip (64 vectors x 1024 rows: 256), and one wave per tile ran
+ * at the issue rate of a single wave, 0.84 us per superblock however the loads were staged; here
+ * a tile keeps four SIMDs busy.
  * MFMA operand layout (16x16x32 i8, checked on gfx950): lane l supplies row (A) / column (B)
  * l % 16 and the 8 K values of group g = l / 16; the result C[4 (l / 16) + j][l % 16] lands in
  * the lane's element j. The 32 columns of a block may be dealt to the K positions in any order
- * that is the same for both operands, since the int32 sum is exact: group g takes the low
- * nibbles of code bytes 4g..4g+3 (columns 4g..4g+3) and their high nibbles (columns
- * 16+4g..16+4g+3), and the staged activations are permuted to the same order. The lane's four
- * result rows are the four rows of tile l / 16, whose 6-bit scales and mins for block k are
- * decoded four at a time (one byte per row). Per (row, vector) the lane then runs
- * acc = fma((float)dot, (D*s)*d, acc); acc = fma(-(M*m), fsum, acc) block by block. */
-template <int NT, int WAVES, int DIST>
-__global__ __launch_bounds__(64 * WAVES) void q4k_mm_k(SegTable tab, int cols, int n,
-                                                       const int8_t *__restrict__ q,
-                                                       const float *__restrict__ d,
-                                                       const float *__restrict__ fs) {
+ * that is the same for both operands, since the int32 sum is exact: group g takes columns 8g ..
+ * 8g + 7, so an activation operand is one 8-byte load and a weight operand the low (g < 2) or high
+ * nibbles of 8 code bytes. Per (row, vector) the lane runs acc = fma((float)dot, (D*s)*d, acc);
+ * acc = fma(-(M*m), fsum, acc) block by block. The MFMA adds to 0x4b400000, the bits of 1.5 * 2^23,
+ * so its result is the float 1.5 * 2^23 + dot (|dot| < 2^22, exact) and a subtraction replaces the
+ * int-to-float conversion, which issues at half the rate.
+ * Bound: 64 vectors of 1024 x 2048 and 1024 x 3584, one load round trip (about 2 us) and a turn of
+ * 0.25 us per superblock: 6.0 and 7.6 us (11.9 and 19.7 us with one wave per tile, which also decoded
+ * the scales once per vector tile); 7168 x 1024 and 8224 x 1024, the rounds of workgroups at two waves
+ * per SIMD: 12.7 and 15.1 us (15.4 and 20.0). */
+constexpr int MM_S = 4;
+
+__global__ __launch_bounds__(64 * MM_S) __attribute__((amdgpu_waves_per_eu(2))) void q4k_mm_k(
+    SegTable tab, int cols, int n, const int8_t *__restrict__ q, const float *__restrict__ d,
+    const float *__restrict__ fs) {
     typedef int v4i __attribute__((ext_vector_type(4)));
-    constexpr int NV16 = NT * 16, T = 64 * WAVES;
-    constexpr int SE = (8 * NV16 + T - 1) / T; /* staged (block, vector) entries per thread */
-    __shared__ __align__(16) uint8_t xs[8 * NV16 * 32]; /* [block][vector][g][8 B] */
-    __shared__ float2 xdf[8 * NV16];                    /* (d, fsum) per [block][vector] */
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int grp_raw = blockIdx.x * WAVES + w; /* 16-row group over all segments */
-    const bool live = grp_raw < tab.total_waves;
-    const int grp = live ? grp_raw : tab.total_waves - 1;
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    /* per wave: the superblock's raw scale lines (4 tiles x 64 bytes), the decoded scales and mins
+     * [block][D s | M m][16 rows], (d, fsum) [block][16 vectors] */
+    __shared__ __align__(16) uint32_t raw_[MM_S][64];
+    __shared__ __align__(16) float scl_[MM_S][8 * 32];
+    __shared__ __align__(16) float2 df_[MM_S][8 * 16];
+    __shared__ __align__(16) float hand[64 * 4]; /* the accumulators between turns */
+    __shared__ int turn;                         /* superblocks whose chains are done */
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c16 = lane & 15, nsb = cols >> 8;
+    const int grp = blockIdx.x; /* 16-row group over all segments */
     const uint8_t *W = tab.s[0].W;
     float *Y = tab.s[0].Y;
     int rows = tab.s[0].rows, ystride = tab.s[0].ystride, grp0 = tab.s[0].wave0;
@@ -817,129 +829,136 @@ __global__ __launch_bounds__(64 * WAVES) void q4k_mm_k(SegTable tab, int cols, i
             ystride = tab.s[t].ystride;
             grp0 = tab.s[t].wave0;
         }
-    const int nsb = cols >> 8;
-    const int row0 = (grp - grp0) * 16;
-    const int vt0 = blockIdx.y * NV16, nvw = n - vt0 < NV16 ? n - vt0 : NV16;
-    const int g = lane >> 4, c16 = lane & 15;
-    /* operand A: row row0 + c16 (clamped into the matrix), code dword g of each block */
-    const int arow = row0 + c16 < rows ? row0 + c16 : rows - 1;
-    const uint8_t *ap = W + (size_t)(arow >> 2) * nsb * SB_BYTES + 64 + 16 * (arow & 3) + 4 * g;
-    /* result rows: tile g of the group (clamped), vector vt0 + 16 t + c16 */
-    const int erow0 = row0 + 4 * g < rows ? row0 + 4 * g : rows - 4;
-    const uint4 *hp = (const uint4 *)(W + (size_t)(erow0 >> 2) * nsb * SB_BYTES);
+    if (tid == 0) turn = 0;
+    __syncthreads();
+    if (w >= nsb) return; /* no superblock of its own; nobody waits for the wave */
+    const int row0 = (grp - grp0) * 16, tile0 = row0 >> 2, tiles = rows >> 2, vt0 = blockIdx.y * 16;
+    const uint32_t tb = (uint32_t)nsb * SB_BYTES;
+    const uint8_t *Wb = W + (size_t)tile0 * tb;
+    /* Byte offsets of the lane's loads within a superblock. Tiles past the matrix and vectors past n
+     * read the last one; their results are not stored. */
+    auto tile_at = [&](int t) { return (uint32_t)(tile0 + t < tiles ? t : tiles - 1 - tile0) * tb; };
+    auto vec_at = [&](int v) { return (uint32_t)(vt0 + v < n ? vt0 + v : n - 1); };
+    const uint32_t oc = tile_at(c16 >> 2) + 64 + 16 * (c16 & 3) + 8 * (g & 1);
+    const uint32_t os = tile_at(lane >> 4) + 4 * (lane & 15);
+    const uint32_t ox = vec_at(c16) * 32 + 8 * g, od = (uint32_t)(g * n) + vec_at(c16);
+    const int sh = 4 * (g >> 1); /* the group's nibbles */
 
-    /* one superblock's inputs; DIST sets, loaded DIST superblocks ahead of their use */
     struct Buf {
-        uint32_t cw[8];
-        uint4 h[4], x0[SE], x1[SE];
-        float2 df[SE];
+        u32x2 c[8], x[8];
+        float d0, d1, f0, f1;
+        uint32_t s;
     };
     auto fetch = [&](Buf &B, int sb) {
+        const uint8_t *wb = Wb + (size_t)sb * SB_BYTES;
+        const int8_t *qb = q + (size_t)sb * 256 * n;
+        const float *db = d + (size_t)sb * 8 * n, *fb = fs + (size_t)sb * 8 * n;
+        B.s = *(const uint32_t *)(wb + os);
+        B.d0 = db[od], B.d1 = db[od + 4 * (uint32_t)n];
+        B.f0 = fb[od], B.f1 = fb[od + 4 * (uint32_t)n];
 #pragma unroll
-        for (int k = 0; k < 8; k++) B.cw[k] = *(const uint32_t *)(ap + (size_t)sb * SB_BYTES + 64 * k);
+        for (int k = 0; k < 8; k++) B.c[k] = *(const u32x2 *)(wb + oc + 64 * k);
 #pragma unroll
-        for (int u = 0; u < 4; u++) B.h[u] = hp[sb * 36 + u];
-#pragma unroll
-        for (int u = 0; u < SE; u++) {
-            const int e = u * T + tid, k = e / NV16, v = e - k * NV16;
-            B.x0[u] = B.x1[u] = make_uint4(0, 0, 0, 0);
-            B.df[u] = make_float2(0.0f, 0.0f);
-            if (e < 8 * NV16 && v < nvw) {
-                const size_t ai = (size_t)(sb * 8 + k) * n + vt0 + v;
-                B.x0[u] = *(const uint4 *)(q + ai * 32);
-                B.x1[u] = *(const uint4 *)(q + ai * 32 + 16);
-                B.df[u] = make_float2(d[ai], fs[ai]);
-            }
-        }
+        for (int k = 0; k < 8; k++) B.x[k] = *(const u32x2 *)(qb + ox + (uint32_t)(k * n) * 32);
     };
 
-    float acc[NT][4];
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[t][j] = 0.0f;
-    const v4i zero = {0, 0, 0, 0};
+    uint8_t *raw = (uint8_t *)raw_[w];
+    float *scl = scl_[w];
+    float2 *df = df_[w];
+    constexpr int BIAS = 0x4b400000; /* the bits of 1.5 * 2^23 */
+    const v4i bias = {BIAS, BIAS, BIAS, BIAS};
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 
-    /* superblock sb from buffer B, whose set is then refilled with superblock sb + DIST */
-    auto step = [&](Buf &B, int sb) {
-        uint32_t cw[8];
+    auto superblock = [&](Buf &B, int sb) {
+        /* the scales: lane = row c16, blocks g and g + 4 (exact: 6-bit x 11-bit) */
+        *(uint32_t *)(raw + 4 * lane) = B.s;
+        df[lane] = make_float2(B.d0, B.f0);
+        df[64 + lane] = make_float2(B.d1, B.f1);
+        __builtin_amdgcn_wave_barrier();
+        {
+            const int i = c16 & 3;
+            const uint8_t *p = raw + 64 * (c16 >> 2);
+            const float D = half_bits_to_float(*(const uint16_t *)(p + 2 * i));
+            const float M = half_bits_to_float(*(const uint16_t *)(p + 8 + 2 * i));
 #pragma unroll
-        for (int k = 0; k < 8; k++) cw[k] = B.cw[k];
-        const uint4 h0 = B.h[0], h1 = B.h[1], h2 = B.h[2], h3 = B.h[3];
-        __syncthreads(); /* the previous superblock's activations are consumed */
-#pragma unroll
-        for (int u = 0; u < SE; u++) {
-            const int e = u * T + tid;
-            if (e < 8 * NV16) {
-                uint2 *dst = (uint2 *)(xs + (size_t)e * 32);
-                dst[0] = make_uint2(B.x0[u].x, B.x1[u].x);
-                dst[1] = make_uint2(B.x0[u].y, B.x1[u].y);
-                dst[2] = make_uint2(B.x0[u].z, B.x1[u].z);
-                dst[3] = make_uint2(B.x0[u].w, B.x1[u].w);
-                xdf[e] = B.df[u];
+            for (int u = 0; u < 2; u++) {
+                const int k = g + 4 * u, j = 4 * k + i;
+                scl[k * 32 + c16] = D * (float)nmx_get6(p + 16, j);
+                scl[k * 32 + 16 + c16] = M * (float)nmx_get6(p + 40, j);
             }
         }
-        if (sb + DIST < nsb) fetch(B, sb + DIST);
-        __syncthreads();
-        float Dj[4], Mj[4];
-        Dj[0] = half_bits_to_float(h0.x), Dj[1] = half_bits_to_float(h0.x >> 16);
-        Dj[2] = half_bits_to_float(h0.y), Dj[3] = half_bits_to_float(h0.y >> 16);
-        Mj[0] = half_bits_to_float(h0.z), Mj[1] = half_bits_to_float(h0.z >> 16);
-        Mj[2] = half_bits_to_float(h0.w), Mj[3] = half_bits_to_float(h0.w >> 16);
-        const uint32_t SL[4] = {h1.x, h1.y, h1.z, h1.w}, SH[2] = {h2.x, h2.y};
-        const uint32_t ML[4] = {h2.z, h2.w, h3.x, h3.y}, MH[2] = {h3.z, h3.w};
+        __builtin_amdgcn_wave_barrier();
+        float fd[8][4], sd[8][4];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            const uint32_t c = cw[k];
-            const long a = (long)(c & 0x0f0f0f0fu) | ((long)((c >> 4) & 0x0f0f0f0fu) << 32);
-            /* 6-bit scale / min of block k for the tile's rows 0..3, one byte each */
-            const int sl = 4 * (k >> 2), sh = 2 * (k >> 1);
-            const uint32_t s4 = ((SL[k & 3] >> sl) & 0x0f0f0f0fu) | (((SH[k & 1] >> sh) & 0x03030303u) << 4);
-            const uint32_t m4 = ((ML[k & 3] >> sl) & 0x0f0f0f0fu) | (((MH[k & 1] >> sh) & 0x03030303u) << 4);
-            float sc[4], of[4];
+            const uint32_t lo = (B.c[k].x >> sh) & 0x0f0f0f0fu, hi = (B.c[k].y >> sh) & 0x0f0f0f0fu;
+            const v4i dot = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                (long)lo | ((long)hi << 32), (long)B.x[k].x | ((long)B.x[k].y << 32), bias, 0, 0, 0);
+            const float4 sc = *(const float4 *)(scl + k * 32 + 4 * g);
+            const float dv = df[k * 16 + c16].x;
+            sd[k][0] = sc.x * dv, sd[k][1] = sc.y * dv, sd[k][2] = sc.z * dv, sd[k][3] = sc.w * dv;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                sc[j] = Dj[j] * (float)((s4 >> (8 * j)) & 0xffu); /* exact: 6-bit x 11-bit */
-                of[j] = Mj[j] * (float)((m4 >> (8 * j)) & 0xffu);
+            for (int j = 0; j < 4; j++) fd[k][j] = __int_as_float(dot[j]) - 12582912.0f;
+        }
+        float4 of[8];
+        float fv[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            of[k] = *(const float4 *)(scl + k * 32 + 16 + 4 * g);
+            fv[k] = df[k * 16 + c16].y;
+        }
+        fetch(B, sb + 2 * MM_S < nsb ? sb + 2 * MM_S : nsb - 1);
+        /* everything above before the turn, so that a turn is the chain alone */
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) asm volatile("" : "+v"(fd[k][j]), "+v"(sd[k][j]));
+            asm volatile("" : "+v"(of[k].x), "+v"(of[k].y), "+v"(of[k].z), "+v"(of[k].w), "+v"(fv[k]));
+        }
+        if (sb > 0) {
+            while (__hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != sb) {
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            const float4 x = *(const float4 *)(hand + 4 * lane);
+            acc[0] = x.x, acc[1] = x.y, acc[2] = x.z, acc[3] = x.w;
+        }
 #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const int e = k * NV16 + 16 * t + c16;
-                const long b = *(const long *)(xs + (size_t)e * 32 + 8 * g);
-                const v4i dot = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, zero, 0, 0, 0);
-                const float2 df = xdf[e];
+        for (int k = 0; k < 8; k++) {
+            const float o[4] = {of[k].x, of[k].y, of[k].z, of[k].w};
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    acc[t][j] = __builtin_fmaf((float)dot[j], sc[j] * df.x, acc[t][j]);
-                    acc[t][j] = __builtin_fmaf(-of[j], df.y, acc[t][j]);
+            for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(fd[k][j], sd[k][j], acc[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(-o[j], fv[k], acc[j]);
+        }
+        if (sb + 1 < nsb) {
+            *(float4 *)(hand + 4 * lane) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (lane == 0)
+                __hip_atomic_store(&turn, sb + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        } else {
+            const int row = row0 + 4 * g, v = vt0 + c16; /* a whole 4-row tile */
+            if (row < rows && v < n) {
+                float *y = Y + (size_t)v * ystride + row;
+                if (((uintptr_t)Y & 15) == 0 && ystride % 4 == 0) {
+                    *(float4 *)y = make_float4(acc[0], acc[1], acc[2], acc[3]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) y[j] = acc[j];
                 }
             }
         }
     };
-
-    if constexpr (DIST == 2) {
-        Buf A, B;
-        fetch(A, 0);
-        if (nsb > 1) fetch(B, 1);
-        for (int sb = 0; sb < nsb; sb += 2) {
-            step(A, sb);
-            if (sb + 1 < nsb) step(B, sb + 1);
-        }
-    } else {
-        Buf A;
-        fetch(A, 0);
-        for (int sb = 0; sb < nsb; sb++) step(A, sb);
+    Buf A, B;
+    fetch(A, w);
+    fetch(B, w + MM_S < nsb ? w + MM_S : nsb - 1);
+    /* whole pairs, so that the sets' loads are outstanding in the same order at every turn and a
+     * wait for one set does not wait for the other */
+    int sb = w;
+    for (; sb + MM_S < nsb; sb += 2 * MM_S) {
+        superblock(A, sb);
+        superblock(B, sb + MM_S);
     }
-    if (!live) return;
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int v = vt0 + 16 * t + c16;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int row = row0 + 4 * g + j;
-            if (v < n && row < rows) Y[(size_t)v * ystride + row] = acc[t][j];
-        }
-    }
+    if (sb < nsb) superblock(A, sb);
 }
 
 /* A8 quantization, one 32-lane half-wave per (block b, vector v) unit; unit index = b * n + v,
@@ -1083,31 +1102,17 @@ int launch_ksplit(nmx_ctx *ctx, const SegTable &tab, int total_rows_groups, int 
     return 0;
 }
 
-/* More than 8 vectors (prefill chunks): the MFMA kernel. Its segment table counts 16-row
- * groups. A wave takes all vector tiles when there are enough row groups to fill the chip,
- * else one tile (four times the waves, the scale decode repeated per tile). */
-int launch_mm(nmx_ctx *ctx, const SegTable &tab, int cols, int n, const int8_t *q,
-              const float *d, const float *fs) {
-    SegTable t16 = tab;
+/* More than 8 vectors (prefill chunks): the MFMA kernel, its segment table counting 16-row groups. */
+int launch_mm(nmx_ctx *ctx, SegTable tab, int cols, int n, const int8_t *q, const float *d,
+              const float *fs) {
     int groups = 0;
     for (int s = 0; s < tab.count; s++) {
-        t16.s[s].wave0 = groups;
+        tab.s[s].wave0 = groups;
         groups += (tab.s[s].rows + 15) / 16;
     }
-    t16.total_waves = groups;
-    const int vtiles = (n + 15) / 16;
-    if (groups < 512) { /* few rows: one vector tile per single-wave workgroup */
-        const dim3 grid((unsigned)groups, (unsigned)vtiles);
-        q4k_mm_k<1, 1, 2><<<grid, 64, 0, ctx->stream>>>(t16, cols, n, q, d, fs);
-    } else {
-        const dim3 grid((unsigned)((groups + 3) / 4));
-        switch (vtiles) {
-        case 4: q4k_mm_k<4, 4, 1><<<grid, 256, 0, ctx->stream>>>(t16, cols, n, q, d, fs); break;
-        case 3: q4k_mm_k<3, 4, 1><<<grid, 256, 0, ctx->stream>>>(t16, cols, n, q, d, fs); break;
-        case 2: q4k_mm_k<2, 4, 1><<<grid, 256, 0, ctx->stream>>>(t16, cols, n, q, d, fs); break;
-        default: q4k_mm_k<1, 4, 1><<<grid, 256, 0, ctx->stream>>>(t16, cols, n, q, d, fs); break;
-        }
-    }
+    tab.total_waves = groups;
+    const dim3 grid((unsigned)groups, (unsigned)((n + 15) / 16));
+    q4k_mm_k<<<grid, 64 * MM_S, 0, ctx->stream>>>(tab, cols, n, q, d, fs);
     NMX_LAUNCHED(ctx, "q4k_mm");
     return 0;
 }
