@@ -139,31 +139,46 @@ __global__ __launch_bounds__(512) void attn_scc_k(Attn a, float *__restrict__ sc
 /* Softmax weights in place, one workgroup per (head, token): max, e_p = exp(s_p - max), the four
  * interleaved partial sums and the tail in order, w_p = e_p * (1 / sum). A segment's exponentials
  * sit in LDS one partial sum after the other (16-byte chain reads); wave 0 adds a segment while
- * waves 1-3 form the next one's, so a long row costs its chain, np / 4 dependent adds. 16.4 us
- * for 512 rows of 4000 positions, 6.6 us on average over a 2000-token prompt. */
-__global__ __launch_bounds__(256) void attn_sm_k(Attn a, float *__restrict__ sc) {
+ * the other waves form the next one's, so a long row costs its chain, np / 4 dependent adds. 512
+ * threads with 8 reads in flight each: 26 us for 8 rows of 20000 positions, 11.5 us for 512 rows of
+ * 4000 (256 threads with one read each: 57.7 and 16.4 us). */
+constexpr int SM_T = 512;
+
+__global__ __launch_bounds__(SM_T) void attn_sm_k(Attn a, float *__restrict__ sc) {
     __shared__ __align__(16) float seg[2][4 * SM_S4 + 4];
     __shared__ float red[8];
     const int tid = threadIdx.x, h = blockIdx.x, t = blockIdx.y;
     const int np = *a.pos + a.pos_off + t + 1;
     float *row = sc + ((size_t)t * a.nh + h) * a.max_ctx;
+    /* f(i, row[i]) for i = i0, i0 + step, .. < end, 8 reads in flight */
+    auto sweep = [&](int i0, int step, int end, auto f) {
+        for (int i = i0; i < end; i += 8 * step) {
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = row[i + u * step < end ? i + u * step : end - 1];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (i + u * step < end) f(i + u * step, x[u]);
+        }
+    };
     float mx = -INFINITY;
-    for (int p = tid; p < np; p += 256) mx = fmaxf(mx, row[p]);
+    sweep(tid, SM_T, np, [&](int, float x) { mx = fmaxf(mx, x); });
     mx = nmx_max_f32_wave(mx);
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    mx = red[0];
+#pragma unroll
+    for (int u = 1; u < SM_T / 64; u++) mx = fmaxf(mx, red[u]);
     const bool many = np > SM_SEG; /* the exponentials of a long row wait in the row itself */
     /* position s0 + i of a segment: partial sum i % 4, its term i / 4 */
     auto exps = [&](int s0, float *dst, int i0, int step) {
-        const int len = np - s0 < SM_SEG ? np - s0 : SM_SEG;
-        for (int i = i0; i < len; i += step) {
-            const float e = nmx_expf_cephes(row[s0 + i] - mx);
-            dst[(i & 3) * SM_S4 + (i >> 2)] = e;
-            if (many) row[s0 + i] = e;
-        }
+        sweep(s0 + i0, step, np - s0 < SM_SEG ? np : s0 + SM_SEG, [&](int p, float x) {
+            const float e = nmx_expf_cephes(x - mx);
+            dst[(p & 3) * SM_S4 + ((p - s0) >> 2)] = e;
+            if (many) row[p] = e;
+        });
     };
-    exps(0, seg[0], tid, 256);
+    exps(0, seg[0], tid, SM_T);
     __syncthreads();
     const int q4 = np & ~3; /* positions in whole quads */
     float chain = 0.0f;     /* lane l < 4: partial sum l; lane 4: the tail */
@@ -175,7 +190,7 @@ __global__ __launch_bounds__(256) void attn_sm_k(Attn a, float *__restrict__ sc)
                 for (int i = full; i < SM_SEG && s0 + i < np; i++)
                     chain = chain + seg[s][(i & 3) * SM_S4 + (i >> 2)];
         } else if (tid >= 64 && s0 + SM_SEG < np) {
-            exps(s0 + SM_SEG, seg[s ^ 1], tid - 64, 192);
+            exps(s0 + SM_SEG, seg[s ^ 1], tid - 64, SM_T - 64);
         }
         __syncthreads();
     }
@@ -183,9 +198,9 @@ __global__ __launch_bounds__(256) void attn_sm_k(Attn a, float *__restrict__ sc)
     __syncthreads();
     const float inv = 1.0f / (((red[0] + red[1]) + (red[2] + red[3])) + red[4]);
     if (many) {
-        for (int p = tid; p < np; p += 256) row[p] = row[p] * inv;
+        sweep(tid, SM_T, np, [&](int p, float e) { row[p] = e * inv; });
     } else {
-        for (int p = tid; p < np; p += 256) row[p] = seg[0][(p & 3) * SM_S4 + (p >> 2)] * inv;
+        for (int p = tid; p < np; p += SM_T) row[p] = seg[0][(p & 3) * SM_S4 + (p >> 2)] * inv;
     }
 }
 
@@ -291,6 +306,77 @@ __global__ __launch_bounds__(512) void attn_pvc_k(const float *__restrict__ wts,
     }
 }
 
+/* P.V of a few rows over a long context (steps and verify passes in caches past 8192 positions),
+ * on the weights of attn_sm_k: workgroup = (32 dims, head, token), wave 0's lanes the chains, one per
+ * dim. The chain, one dependent add per position, bounds it (8.1 clocks a step: 68 us for 20000
+ * positions), so everything else runs beside it: waves 1-4 store tile i + 1's products w_p v_p[d] in
+ * LDS, one row per dim, while wave 0 adds tile i, and have tile i + 2's values and weights in flight.
+ * One token at 20000 positions, binary16 cache: 93 us
+ * (attn_sm_k before it 26 us; one kernel that formed the weights twice and stored each tile between
+ * two chains: 429 us). */
+constexpr int PL_P = 256;        /* positions per tile */
+constexpr int PL_D = 32;         /* output dims per workgroup: one A8 block */
+constexpr int PL_RS = PL_P + 4;  /* row stride: 16-byte aligned, 4 words apart modulo 64 banks */
+
+template <int KVT>
+__global__ __launch_bounds__(320) void attn_pvl_k(const float *__restrict__ wts, Attn a) {
+    constexpr int F4 = PL_D / 4, PER = PL_P * F4 / 256;
+    __shared__ __align__(16) float vt[2][PL_D * PL_RS];
+    const int hd = a.hd, rep = a.nh / a.nkv, S = (hd / PL_D) * a.nkv, tid = threadIdx.x;
+    const int sl = blockIdx.x % S, k = blockIdx.x / S; /* a slice of V to one XCD, as attn_pvc_k */
+    const int d0 = (sl % (hd / PL_D)) * PL_D, g = sl / (hd / PL_D);
+    const int h = g * rep + k % rep, t = k / rep;
+    const int np = *a.pos + a.pos_off + t + 1, ntile = (np + PL_P - 1) / PL_P;
+    const size_t R0 = (size_t)g * a.max_ctx;
+    const float *vsc = kv_scales<KVT>(a.vc, a);
+    const float *wr = wts + ((size_t)t * a.nh + h) * a.max_ctx;
+    if (tid >= 64) { /* waves 1-4: 8 lanes to a position */
+        const int f0 = tid - 64, c4 = f0 % F4, r0 = f0 / F4;
+        float4 v[PER];
+        float w[PER];
+        auto fetch = [&](int i) { /* clamped: positions past the row are stored and never added */
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                int p = i * PL_P + u * (256 / F4) + r0;
+                p = p < np ? p : np - 1;
+                v[u] = kv_load4<KVT>(a.vc, R0 + p, hd, d0 + 4 * c4, vsc);
+                w[u] = wr[p];
+            }
+        };
+        fetch(0);
+        for (int i = 0; i < ntile; i++) {
+            float *q = vt[i & 1] + 4 * c4 * PL_RS + r0;
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                float *x = q + u * (256 / F4);
+                x[0] = w[u] * v[u].x;
+                x[PL_RS] = w[u] * v[u].y;
+                x[2 * PL_RS] = w[u] * v[u].z;
+                x[3 * PL_RS] = w[u] * v[u].w;
+            }
+            fetch(i + 1);
+            __syncthreads(); /* tile i stored; tile i - 1 added */
+        }
+        return;
+    }
+    const float gate = tid < PL_D ? a.q[((size_t)t * a.nh + h) * 2 * hd + hd + d0 + tid] : 0.0f;
+    float o = 0.0f;
+    for (int i = 0; i < ntile; i++) {
+        __syncthreads();
+        const int rows = np - i * PL_P < PL_P ? np - i * PL_P : PL_P;
+        if (tid < PL_D) o = pv_chain4(o, vt[i & 1] + tid * PL_RS, rows);
+    }
+    if (tid < PL_D) {
+        o = o * nmx_sigmoid(gate);
+        const int col = h * hd + d0 + tid;
+        a.o[(size_t)t * a.nh * hd + col] = o;
+        if (a.aq) {
+            const size_t u = (size_t)(col >> 5) * a.an + t;
+            nmx_a8_store(o, a.aq + u * 32, a.ad + u, a.afs + u);
+        }
+    }
+}
+
 template <int KVT>
 int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
     const int rows = a.n * (a.nh / a.nkv);
@@ -306,7 +392,7 @@ int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
                      (unsigned)((rows + SC_ROWS - 1) / SC_ROWS), (unsigned)a.nkv);
     attn_scc_k<KVT><<<sgrid, 512, lds, ctx->stream>>>(a, sc);
     NMX_LAUNCHED(ctx, "attn_scc");
-    attn_sm_k<<<dim3((unsigned)a.nh, (unsigned)a.n), 256, 0, ctx->stream>>>(a, sc);
+    attn_sm_k<<<dim3((unsigned)a.nh, (unsigned)a.n), SM_T, 0, ctx->stream>>>(a, sc);
     NMX_LAUNCHED(ctx, "attn_sm");
     const unsigned pg = (unsigned)((a.hd / PV_D) * a.nkv * ((rows + PV_W - 1) / PV_W));
     attn_pvc_k<KVT><<<pg, 512, 0, ctx->stream>>>(sc, a);
@@ -315,6 +401,17 @@ int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
 }
 
 } // namespace
+
+int nmx_attn_long(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, float *sc) {
+    attn_sm_k<<<dim3((unsigned)a.nh, (unsigned)a.n), SM_T, 0, ctx->stream>>>(a, sc);
+    NMX_LAUNCHED(ctx, "attn_sm");
+    const unsigned pg = (unsigned)((a.hd / PL_D) * a.nh * a.n);
+    if (kv_dtype == KV_F16) attn_pvl_k<KV_F16><<<pg, 320, 0, ctx->stream>>>(sc, a);
+    else if (kv_dtype == KV_I8) attn_pvl_k<KV_I8><<<pg, 320, 0, ctx->stream>>>(sc, a);
+    else attn_pvl_k<KV_F32><<<pg, 320, 0, ctx->stream>>>(sc, a);
+    NMX_LAUNCHED(ctx, "attn_pvl");
+    return 0;
+}
 
 int nmx_attn_chunk(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, float *sc) {
     if (kv_dtype == KV_F16) return launch_chunk<KV_F16>(ctx, a, sc);

@@ -996,78 +996,8 @@ __global__ __launch_bounds__(256) void attn_pv_k(const float *__restrict__ sc,
     }
 }
 
-/* The same softmax and P.V for caches longer than the scores row that fits in LDS (max_ctx
- * above PV_ATT_MAX): the max over the row from the scores workspace, then the exponentials
- * segment by segment (SEG positions in LDS) with the four ordered partial sums and the tail
- * carried across segments, then the value rows in tiles, each weight recomputed as
- * e_p * (1 / sum) with e_p = exp(s_p - max) (the same operations as the in-LDS kernel, so the
- * results are identical). */
 constexpr int PV_ATT_MAX = 8192; /* scores kept in LDS by attn_pv_k */
-constexpr int PV_SEG = 4096;     /* positions per exponential segment of attn_pv_long_k */
-
-template <int KVT>
-__global__ __launch_bounds__(256) void attn_pv_long_k(Attn a, const float *__restrict__ sc) {
-    extern __shared__ float4 smem4[];
-    __shared__ float red[8];
-    constexpr int F4 = PV_DS / 4;
-    const int hd = a.hd, rep = a.nh / a.nkv, S = (hd / PV_DS) * a.nkv;
-    const int tid = threadIdx.x, sl = blockIdx.x % S, k = blockIdx.x / S;
-    const int d0 = (sl % (hd / PV_DS)) * PV_DS, g = sl / (hd / PV_DS);
-    const int h = g * rep + k % rep, t = k / rep;
-    const int np = *a.pos + a.pos_off + t + 1;
-    float *seg = (float *)smem4;     /* [PV_SEG] */
-    float *vt = seg + PV_SEG;        /* [PV_PT2][PV_DS] */
-    const float *srow = sc + ((size_t)t * a.nh + h) * a.max_ctx;
-    const size_t R0 = (size_t)g * a.max_ctx;
-    const float *vsc = kv_scales<KVT>(a.vc, a);
-
-    float mx = -INFINITY;
-    for (int p = tid; p < np; p += 256) mx = fmaxf(mx, srow[p]);
-    mx = nmx_max_f32_wave(mx);
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    __syncthreads();
-
-    /* partial sum l over e[4m + l], m ascending (m < np / 4), and the tail, in order */
-    const int q4 = 4 * (np >> 2);
-    float chain = 0.0f; /* lane tid < 4: partial sum tid; lane 4: the tail */
-    for (int s0 = 0; s0 < np; s0 += PV_SEG) {
-        const int len = np - s0 < PV_SEG ? np - s0 : PV_SEG;
-        for (int p = tid; p < len; p += 256) seg[p] = nmx_expf_cephes(srow[s0 + p] - mx);
-        __syncthreads();
-        const int full = q4 - s0 < len ? (q4 - s0 > 0 ? q4 - s0 : 0) : len; /* in quads' range */
-        if (tid < 4) chain = pv_chain(chain, seg + tid, 4, full >> 2);
-        else if (tid == 4)
-            for (int i = full; i < len; i++) chain = chain + seg[i];
-        __syncthreads();
-    }
-    if (tid < 5) red[tid] = chain;
-    __syncthreads();
-    const float inv = 1.0f / (((red[0] + red[1]) + (red[2] + red[3])) + red[4]);
-
-    float o = 0.0f;
-    for (int base = 0; base < np; base += PV_PT2) {
-        const int rows = np - base < PV_PT2 ? np - base : PV_PT2;
-        for (int f = tid; f < rows * F4; f += 256) {
-            const int r = f / F4, c4 = f - r * F4;
-            const float4 v = kv_load4<KVT>(a.vc, R0 + base + r, hd, d0 + 4 * c4, vsc);
-            const float w = nmx_expf_cephes(srow[base + r] - mx) * inv;
-            *(float4 *)(vt + r * PV_DS + 4 * c4) = make_float4(w * v.x, w * v.y, w * v.z, w * v.w);
-        }
-        __syncthreads();
-        if (tid < PV_DS) o = pv_chain(o, vt + tid, PV_DS, rows);
-        __syncthreads();
-    }
-    if (tid < PV_DS) {
-        const int d = d0 + tid;
-        const float *qrow = a.q + ((size_t)t * a.nh + h) * 2 * hd;
-        o = o * nmx_sigmoid(qrow[hd + d]);
-        const int col = h * hd + d;
-        a.o[(size_t)t * a.nh * hd + col] = o;
-        if (a.aq) a8_block(o, col >> 5, t, a.n, a.aq, a.ad, a.afs);
-    }
-}
+constexpr int PV_SEG = 4096;     /* exponentials per segment of top1_gate_k */
 
 /* ---- confidence gate of a draft (engine/src/spec.c:93-97, forward_ops.c:294-353) -------
  * p = 1 / s, s = sum of e_i = pf_expf(l_i - max) in the reference's order; flag = p >= tau.
@@ -1575,6 +1505,8 @@ int launch_attn(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
 
 template <int KVT>
 int launch_pv(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
+    /* score rows past the LDS go through memory as softmax weights */
+    if (p->max_ctx > PV_ATT_MAX) return nmx_attn_long(ctx, a, KVT, p->scores);
     const unsigned pgrid = (unsigned)((p->hd / PV_DS) * p->nh * p->n);
     const size_t plds = ((size_t)4 * cm_stride(p->max_ctx) + 4 + (size_t)PV_DS * PV_RS) * 4;
     static bool pv_ready = false; /* idempotent */
@@ -1585,13 +1517,8 @@ int launch_pv(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
                                                 (size_t)PV_DS * PV_RS) * 4)));
         pv_ready = true;
     }
-    if (p->max_ctx > PV_ATT_MAX) {
-        const size_t llds = ((size_t)PV_SEG + (size_t)PV_PT2 * PV_DS) * 4;
-        attn_pv_long_k<KVT><<<pgrid, 256, llds, ctx->stream>>>(a, p->scores);
-    } else {
-        attn_pv_k<KVT><<<pgrid, 256, plds, ctx->stream>>>(p->scores, a.pos, a.vc, a.pos_off, a.max_ctx,
-                                                           a.nh, a.nkv, a.hd, a);
-    }
+    attn_pv_k<KVT><<<pgrid, 256, plds, ctx->stream>>>(p->scores, a.pos, a.vc, a.pos_off, a.max_ctx,
+                                                       a.nh, a.nkv, a.hd, a);
     NMX_LAUNCHED(ctx, "attn_pv");
     return 0;
 }

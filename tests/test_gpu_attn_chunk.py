@@ -82,3 +82,46 @@ def test_chunk_equals_steps(dev, case):
     got = passes(dev, host, case, 64)
     for k in want:
         assert_bits_equal(got[k], want[k], k)
+
+
+def widen(cache, kvt, nkv, ctx, wide, hd):
+    """The cache's rows in a cache of `wide` positions per head."""
+    size = (4, 2, 1)[kvt] * hd
+    rows = np.zeros((nkv, wide, size), np.uint8)
+    rows[:, :ctx] = cache[:nkv * ctx * size].reshape(nkv, ctx, size)
+    if kvt != 2:
+        return rows.ravel()
+    scales = np.zeros((nkv, wide), np.float32)
+    scales[:, :ctx] = cache[nkv * ctx * size:].view(np.float32).reshape(nkv, ctx)
+    return np.concatenate([rows.ravel(), scales.ravel().view(np.uint8)])
+
+
+@pytest.mark.parametrize("case", [
+    # n, query heads, KV heads, head size, kv dtype, position of token 0
+    (1, 8, 2, 256, 1, 8000), (5, 8, 2, 256, 0, 4094), (8, 4, 4, 64, 2, 250), (3, 6, 2, 128, 0, 0),
+    (1, 8, 2, 256, 2, 255), (2, 8, 2, 256, 0, 511),
+], ids=lambda c: "n%d_h%d_%d_hd%d_kv%d_pos%d" % c)
+def test_long_cache_equals_in_lds(dev, case):
+    """A cache past 8192 positions (softmax weights through memory, P.V products made beside the
+    chains in 256-position tiles) against the same rows in one of 8192 (attn_pv_k)."""
+    n, nh, nkv, hd, kvt, pos0 = case
+    print(f"[case] attn long {case}", flush=True)
+    ctx, wide = 8192, 8200
+    rng = np.random.default_rng(n + hd + pos0)
+    ang = rng.uniform(0, 2 * np.pi, (wide, hd // 8))
+    host = dict(
+        q=rng.standard_normal((n, nh, 2 * hd)).astype(np.float32),
+        k_in=rng.standard_normal((n, nkv * hd)).astype(np.float32),
+        v_in=rng.standard_normal((n, nkv * hd)).astype(np.float32),
+        q_norm=rng.uniform(0.5, 1.5, hd).astype(np.float32),
+        k_norm=rng.uniform(0.5, 1.5, hd).astype(np.float32),
+        cos=np.cos(ang).astype(np.float32), sin=np.sin(ang).astype(np.float32),
+        kc=cache_bytes(rng, kvt, nkv, ctx, hd), vc=cache_bytes(rng, kvt, nkv, ctx, hd),
+    )
+    want = passes(dev, host, (n, nh, nkv, hd, ctx, kvt, pos0), 8)
+    far = dict(host, **{c: widen(host[c], kvt, nkv, ctx, wide, hd) for c in ("kc", "vc")})
+    got = passes(dev, far, (n, nh, nkv, hd, wide, kvt, pos0), 8)
+    for k in ("o", "aq", "ad", "afs"):
+        assert_bits_equal(got[k], want[k], k)
+    for k in ("kc", "vc"):
+        assert_bits_equal(got[k], widen(want[k], kvt, nkv, ctx, wide, hd), k)
