@@ -423,6 +423,29 @@ int nmx_attn(nmx_ctx *ctx, const nmx_attn_args *p);
  * and at most 8 tokens, else the two calls. */
 int nmx_attn_fused(nmx_ctx *ctx, const nmx_attn_args *p);
 
+/* ---- prompts in larger chunks -------------------------------------------------------------
+ * The calls of one forward pass for up to NMX_CHUNK_ROWS rows at once, each as the call without
+ * the suffix in everything else (arguments, layouts, results bit for bit: no result depends on the
+ * rows it shares a launch with). No counterpart in the reference, whose chunks have at most 64
+ * rows; a longer chunk fills the device and spreads a layer's launches over more tokens.
+ * nmx_q4k_matmul_chunk is nmx_q4k_matmul_multi. nmx_lin_mix_chunk: above 64 rows only without a
+ * log, in the shapes of nmx_lin_chunk_ok (1 if they take it; host only) and with every intermediate
+ * buffer given. nmx_attn_fused_chunk: the scores workspace holds score_rows rows, [score_rows][nh]
+ * [max_ctx] floats. */
+#define NMX_CHUNK_ROWS 512
+int nmx_q4k_matmul_chunk(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                         float *const *Y, const int *y_stride, int cols, int n, const int8_t *q,
+                         const float *d, const float *fsum);
+int nmx_q4k_matmul_norm_chunk(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                              float *const *Y, const int *y_stride, int cols, int n,
+                              const nmx_norm_in *in, nmx_a8 a8_tmp);
+int nmx_q4k_swiglu_chunk(nmx_ctx *ctx, const void *Wg, const void *Wu, int ffn, int cols, int n,
+                         const int8_t *q, const float *d, const float *fsum, const nmx_norm_in *in,
+                         float *y, nmx_a8 out, nmx_a8 a8_tmp, float *gate_tmp, float *up_tmp);
+int nmx_lin_mix_chunk(nmx_ctx *ctx, const nmx_lin_mix_args *a);
+int nmx_lin_chunk_ok(int dk, int dv, int conv_k, int heads);
+int nmx_attn_fused_chunk(nmx_ctx *ctx, const nmx_attn_args *p, int score_rows);
+
 /* The reference's chain gate (engine/src/spec_adapt.c:56, spec.c:89-97) as a device op, for a
  * caller that drives the reference's own confidence-gated adaptive chain on this device layer;
  * the engine's own adaptive policy (pinfer_spec_params.adaptive) decides on the host and does

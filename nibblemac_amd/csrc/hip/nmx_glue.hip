@@ -1463,8 +1463,8 @@ int nmx_silu_mul(nmx_ctx *ctx, const float *gate, const float *up, int stride, i
     return 0;
 }
 
-static int attn_args(nmx_ctx *ctx, const nmx_attn_args *p, Attn *a) {
-    if (!p || p->n < 1 || p->n > 64 || p->nkv < 1 || p->nh < p->nkv || p->nh % p->nkv ||
+static int attn_args(nmx_ctx *ctx, const nmx_attn_args *p, Attn *a, int nmax = 64) {
+    if (!p || p->n < 1 || p->n > nmax || p->nkv < 1 || p->nh < p->nkv || p->nh % p->nkv ||
         p->hd < 64 || p->hd > 512 || p->hd % 64 || p->rot % 2 || p->rot > p->hd ||
         p->max_ctx < 1 || p->max_ctx > (1 << 20) || !p->q || !p->k_in || !p->v_in || !p->q_norm ||
         !p->k_norm || !p->rope_cos || !p->rope_sin || !p->kc || !p->vc || !p->pos || !p->o)
@@ -1560,6 +1560,30 @@ int nmx_attn_fused(nmx_ctx *ctx, const nmx_attn_args *p) {
     if (p->kv_dtype == KV_F16) return launch_attn_fused<KV_F16>(ctx, p, a);
     if (p->kv_dtype == KV_I8) return launch_attn_fused<KV_I8>(ctx, p, a);
     return launch_attn_fused<KV_F32>(ctx, p, a);
+}
+
+int nmx_attn_fused_chunk(nmx_ctx *ctx, const nmx_attn_args *p, int score_rows) {
+    if (!ctx) return -1;
+    if (p && p->n <= 64 && p->n <= score_rows) return nmx_attn_fused(ctx, p);
+    Attn a;
+    if (attn_args(ctx, p, &a, NMX_CHUNK_ROWS)) return -1;
+    if (!p->scores || score_rows < 1)
+        return nmx_fail(ctx, "nmx_attn_fused_chunk: NULL scores workspace");
+    if (p->kv_dtype == KV_F16) launch_attn_prep<KV_F16>(ctx, p, a);
+    else if (p->kv_dtype == KV_I8) launch_attn_prep<KV_I8>(ctx, p, a);
+    else launch_attn_prep<KV_F32>(ctx, p, a);
+    NMX_LAUNCHED(ctx, "attn_prep");
+    /* the workspace's rows at a time; a row's bits do not depend on the others */
+    for (int t0 = 0; t0 < p->n; t0 += score_rows) {
+        Attn b = a;
+        b.n = p->n - t0 < score_rows ? p->n - t0 : score_rows;
+        b.q += (size_t)t0 * a.nh * 2 * a.hd;
+        b.o += (size_t)t0 * a.nh * a.hd;
+        b.pos_off += t0;
+        if (b.aq) b.aq += (size_t)t0 * 32, b.ad += t0, b.afs += t0;
+        if (nmx_attn_chunk(ctx, b, p->kv_dtype, p->scores)) return -1;
+    }
+    return 0;
 }
 
 int nmx_attn_prep(nmx_ctx *ctx, const nmx_attn_args *p) {

@@ -452,7 +452,7 @@ bool chunk_ok(const nmx_lin_mix_args &a) {
     const nmx_lin_args &r = a.rule;
     if (!nmx_lin_rulec_ok(r) || p.conv_k != 4 || p.xin || p.dk > 256 || p.C % 32 || r.heads < 1 ||
         r.heads > 256 || r.rep < 1 || r.heads % r.rep || r.dv < 32 || r.dv > 512 || r.keep < 0 ||
-        r.keep > 64 || (r.keep > 0 && !r.pend) || p.n * p.heads > 4096 || !p.raw || !p.state ||
+        r.keep > 64 || (r.keep > 0 && !r.pend) || !p.raw || !p.state ||
         !p.conv_w || !p.b_in || !p.a_in || !p.dt_bias || (!p.A_log && !p.A) || !p.out || !p.beta ||
         !p.decay || !r.S || !r.o || p.raw_stride < p.C || p.g_stride < p.heads)
         return false;
@@ -488,13 +488,13 @@ bool chunk_ok(const nmx_lin_mix_args &a) {
 
 extern "C" {
 
-int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) {
+static int lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a, int nmax) {
     if (!ctx) return -1;
     if (!a) return nmx_fail(ctx, "nmx_lin_mix: NULL args");
     const nmx_lin_pre_args &p = a->pre;
     const nmx_lin_args &r = a->rule;
     const int n = p.n, dk = p.dk, dv = r.dv;
-    if (n < 1 || n > 64 || n != r.n || dk != r.dk || p.heads != r.heads || !a->z || !a->norm_w ||
+    if (n < 1 || n > nmax || n != r.n || dk != r.dk || p.heads != r.heads || !a->z || !a->norm_w ||
         a->z_stride < r.heads * dv || (a->y && a->y_stride < r.heads * dv) || dv % 32 ||
         p.kd != (r.heads / r.rep) * dk || p.C != 2 * p.kd + r.heads * dv)
         return nmx_fail(ctx, "nmx_lin_mix: inconsistent arguments");
@@ -516,6 +516,7 @@ int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) {
         return nmx_lin_post(ctx, r.o, r.o_stride, a->z, a->z_stride, a->norm_w, n, r.heads, dv,
                             a->eps, a->y, a->y_stride, a->a8);
     }
+    if (n > 64) return nmx_fail(ctx, "nmx_lin_mix_chunk: n=%d outside the chunk kernels' limits", n);
     if (!fused) { /* the separate kernels, through the intermediate buffers of the structs */
         if (nmx_lin_pre(ctx, &p) || nmx_lin_rule(ctx, &r)) return -1;
         return nmx_lin_post(ctx, r.o, r.o_stride, a->z, a->z_stride, a->norm_w, n, r.heads, dv,
@@ -530,6 +531,17 @@ int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) {
              r.S, r.log, r.pend, r.keep, r.log0, r.keep_dev, a->z, a->z_stride, a->norm_w,
              a->eps, a->y, a->y_stride, a->a8.q, a->a8.d, a->a8.fs};
     return dk == 64 ? launch_mix<16>(ctx, m, lds) : launch_mix<32>(ctx, m, lds);
+}
+
+int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) { return lin_mix(ctx, a, 64); }
+
+int nmx_lin_mix_chunk(nmx_ctx *ctx, const nmx_lin_mix_args *a) {
+    return lin_mix(ctx, a, NMX_CHUNK_ROWS);
+}
+
+int nmx_lin_chunk_ok(int dk, int dv, int conv_k, int heads) {
+    return (dk == 64 || dk == 128 || dk == 256) && dv >= 32 && dv <= 512 && dv % 32 == 0 &&
+           conv_k == 4 && heads >= 1 && heads <= 256;
 }
 
 } /* extern "C" */

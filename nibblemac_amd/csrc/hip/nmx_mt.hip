@@ -949,12 +949,12 @@ int nmx_mt_plan(int count, const int *rows, int cols, int n, int norm, int swigl
     return rc;
 }
 
-int nmx_q4k_matmul_norm(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
-                        float *const *Y, const int *y_stride, int cols, int n,
-                        const nmx_norm_in *in, nmx_a8 a8_tmp) {
+static int matmul_norm(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                       float *const *Y, const int *y_stride, int cols, int n,
+                       const nmx_norm_in *in, nmx_a8 a8_tmp, int nmax) {
     if (!ctx) return -1;
     if (!in || !in->x || !in->w || count < 1 || count > NMX_MAX_SEGS || !W || !rows || !Y ||
-        !y_stride || cols <= 0 || cols % 256 || cols > 65536 || n < 1 || n > 64 ||
+        !y_stride || cols <= 0 || cols % 256 || cols > 65536 || n < 1 || n > nmax ||
         in->x_stride < cols || (in->add && in->add_stride < cols) ||
         (in->x_out && in->xo_stride < cols))
         return nmx_fail(ctx, "nmx_q4k_matmul_norm: bad arguments");
@@ -987,8 +987,20 @@ int nmx_q4k_matmul_norm(nmx_ctx *ctx, int count, const void *const *W, const int
     if (nmx_rmsnorm_xo(ctx, in->x, in->x_stride, in->add, in->add_stride, in->x_out,
                        in->xo_stride, in->w, n, cols, in->eps, nullptr, 0, a8_tmp))
         return -1;
-    return nmx_q4k_matmul_multi(ctx, count, W, rows, Y, y_stride, cols, n, a8_tmp.q, a8_tmp.d,
+    return nmx_q4k_matmul_chunk(ctx, count, W, rows, Y, y_stride, cols, n, a8_tmp.q, a8_tmp.d,
                                 a8_tmp.fs);
+}
+
+int nmx_q4k_matmul_norm(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                        float *const *Y, const int *y_stride, int cols, int n,
+                        const nmx_norm_in *in, nmx_a8 a8_tmp) {
+    return matmul_norm(ctx, count, W, rows, Y, y_stride, cols, n, in, a8_tmp, 64);
+}
+
+int nmx_q4k_matmul_norm_chunk(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                              float *const *Y, const int *y_stride, int cols, int n,
+                              const nmx_norm_in *in, nmx_a8 a8_tmp) {
+    return matmul_norm(ctx, count, W, rows, Y, y_stride, cols, n, in, a8_tmp, NMX_CHUNK_ROWS);
 }
 
 int nmx_q4k_matmul_embed_norm(nmx_ctx *ctx, const void *W, int rows, float *Y, int y_stride,
@@ -1028,12 +1040,12 @@ int nmx_q4k_matmul_embed_norm(nmx_ctx *ctx, const void *W, int rows, float *Y, i
                           nullptr);
 }
 
-int nmx_q4k_swiglu(nmx_ctx *ctx, const void *Wg, const void *Wu, int ffn, int cols, int n,
-                   const int8_t *q, const float *d, const float *fsum, const nmx_norm_in *in,
-                   float *y, nmx_a8 out, nmx_a8 a8_tmp, float *gate_tmp, float *up_tmp) {
+static int swiglu_n(nmx_ctx *ctx, const void *Wg, const void *Wu, int ffn, int cols, int n,
+                    const int8_t *q, const float *d, const float *fsum, const nmx_norm_in *in,
+                    float *y, nmx_a8 out, nmx_a8 a8_tmp, float *gate_tmp, float *up_tmp, int nmax) {
     if (!ctx) return -1;
     if (!Wg || !Wu || ffn <= 0 || ffn % 32 || cols <= 0 || cols % 256 || cols > 65536 || n < 1 ||
-        n > 64 || !out.q || !out.d || !out.fs || (!in && (!q || !d || !fsum)) ||
+        n > nmax || !out.q || !out.d || !out.fs || (!in && (!q || !d || !fsum)) ||
         (in && (!in->x || !in->w || in->x_stride < cols || (in->add && in->add_stride < cols) ||
                 (in->x_out && in->xo_stride < cols))))
         return nmx_fail(ctx, "nmx_q4k_swiglu: bad arguments");
@@ -1056,8 +1068,21 @@ int nmx_q4k_swiglu(nmx_ctx *ctx, const void *Wg, const void *Wu, int ffn, int co
     const void *W[2] = {Wg, Wu};
     const int R[2] = {ffn, ffn};
     float *Y[2] = {gate_tmp, up_tmp};
-    if (nmx_q4k_matmul_multi(ctx, 2, W, R, Y, R, cols, n, q, d, fsum)) return -1;
+    if (nmx_q4k_matmul_chunk(ctx, 2, W, R, Y, R, cols, n, q, d, fsum)) return -1;
     return nmx_silu_mul(ctx, gate_tmp, up_tmp, ffn, n, ffn, y, out);
+}
+
+int nmx_q4k_swiglu(nmx_ctx *ctx, const void *Wg, const void *Wu, int ffn, int cols, int n,
+                   const int8_t *q, const float *d, const float *fsum, const nmx_norm_in *in,
+                   float *y, nmx_a8 out, nmx_a8 a8_tmp, float *gate_tmp, float *up_tmp) {
+    return swiglu_n(ctx, Wg, Wu, ffn, cols, n, q, d, fsum, in, y, out, a8_tmp, gate_tmp, up_tmp, 64);
+}
+
+int nmx_q4k_swiglu_chunk(nmx_ctx *ctx, const void *Wg, const void *Wu, int ffn, int cols, int n,
+                         const int8_t *q, const float *d, const float *fsum, const nmx_norm_in *in,
+                         float *y, nmx_a8 out, nmx_a8 a8_tmp, float *gate_tmp, float *up_tmp) {
+    return swiglu_n(ctx, Wg, Wu, ffn, cols, n, q, d, fsum, in, y, out, a8_tmp, gate_tmp, up_tmp,
+                    NMX_CHUNK_ROWS);
 }
 
 } /* extern "C" */

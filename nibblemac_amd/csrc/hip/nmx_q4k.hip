@@ -1212,14 +1212,14 @@ int nmx_quant_a8(nmx_ctx *ctx, const float *X, int n, int cols, int8_t *q, float
     return 0;
 }
 
-int nmx_q4k_matmul_multi(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
-                         float *const *Y, const int *y_stride, int cols, int n,
-                         const int8_t *q, const float *d, const float *fsum) {
+static int matmul_multi(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                        float *const *Y, const int *y_stride, int cols, int n, const int8_t *q,
+                        const float *d, const float *fsum, int nmax) {
     if (!ctx) return -1;
     if (count < 1 || count > NMX_MAX_SEGS || !W || !rows || !Y || !y_stride)
         return nmx_fail(ctx, "nmx_q4k_matmul_multi: bad segment list (count=%d)", count);
     if (!q || !d || !fsum) return nmx_fail(ctx, "nmx_q4k_matmul: NULL activation pointer");
-    if (cols <= 0 || cols % 256 || cols > 65536 || n < 1 || n > 64)
+    if (cols <= 0 || cols % 256 || cols > 65536 || n < 1 || n > nmax)
         return nmx_fail(ctx, "nmx_q4k_matmul: bad shape cols=%d n=%d", cols, n);
     const size_t qb = (size_t)n * cols, fb = (size_t)n * (cols / 32) * 4;
     SegTable tab = {};
@@ -1239,6 +1239,18 @@ int nmx_q4k_matmul_multi(nmx_ctx *ctx, int count, const void *const *W, const in
     }
     tab.total_waves = waves;
     return launch_passes(ctx, tab, cols, n, q, d, fsum, nullptr);
+}
+
+int nmx_q4k_matmul_multi(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                         float *const *Y, const int *y_stride, int cols, int n,
+                         const int8_t *q, const float *d, const float *fsum) {
+    return matmul_multi(ctx, count, W, rows, Y, y_stride, cols, n, q, d, fsum, 64);
+}
+
+int nmx_q4k_matmul_chunk(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
+                         float *const *Y, const int *y_stride, int cols, int n,
+                         const int8_t *q, const float *d, const float *fsum) {
+    return matmul_multi(ctx, count, W, rows, Y, y_stride, cols, n, q, d, fsum, NMX_CHUNK_ROWS);
 }
 
 int nmx_q4k_matmul(nmx_ctx *ctx, const void *W, int rows, int cols, int n, const int8_t *q,

@@ -84,7 +84,18 @@ static int rope_tables(pinfer_ctx *c, int *ok) {
 
 static int alloc_state(pinfer_ctx *c) {
     int ok = 1;
-    const int B = E_MAX_BATCH, H = c->H, S = c->conv_k - 1;
+    /* a prompt's chunk: 512 rows, or 64 where the DeltaNet chunk kernels do not take the shape; no
+     * more than a context holds, rounded up to whole passes of 64 */
+    const int fit = (c->max_ctx + 63) / 64 * 64;
+    c->chunk = !c->n_lin || nmx_lin_chunk_ok(c->lk_dim, c->lv_dim, c->conv_k, c->lv_heads) ? E_CHUNK : 64;
+    if (c->chunk > fit) c->chunk = fit;
+    /* attention takes the chunk in slices of the scores workspace's rows: 64 to 256 (more rows fill
+     * the device at shorter contexts), at most E_SCORE_BYTES above 64 */
+    const size_t row = (size_t)imax(c->n_heads, 1) * c->max_ctx * 4;
+    c->score_rows = E_SCORE_BYTES / row > 256 ? 256 : (int)(E_SCORE_BYTES / row) / 64 * 64;
+    if (c->score_rows < 64) c->score_rows = 64;
+    if (c->score_rows > c->chunk) c->score_rows = c->chunk;
+    const int B = c->chunk, H = c->H, S = c->conv_k - 1;
     const size_t logw = (size_t)c->lk_dim + c->lv_dim + 1;
     c->cap = E_MAX_K + 1;
     c->conv_state = dalloc(c, (size_t)imax(c->n_lin, 1) * (S ? S : 1) * c->conv_dim * 4, &ok);
@@ -119,14 +130,14 @@ static int alloc_state(pinfer_ctx *c) {
     s->decay = dalloc(c, (size_t)B * c->lv_heads * 4, &ok);
     s->cat = dalloc(c, (size_t)B * 2 * H * 4, &ok);
     s->emb = dalloc(c, (size_t)B * H * 4, &ok);
-    s->sc = dalloc(c, (size_t)B * imax(c->n_heads, 1) * c->max_ctx * 4, &ok);
+    s->sc = dalloc(c, (size_t)c->score_rows * row, &ok);
     s->row1 = dalloc(c, (size_t)H * 4, &ok);
     s->a_h = a8_alloc(c, H, B, &ok);
     s->a_w = a8_alloc(c, wide, B, &ok);
     s->a_f = a8_alloc(c, c->ffn, B, &ok);
     s->a_1 = a8_alloc(c, H, 1, &ok);
     c->hbuf = dalloc(c, (size_t)B * H * 4, &ok);
-    c->pbuf = dalloc(c, (size_t)B * H * 4, &ok);
+    c->pbuf = dalloc(c, (size_t)E_MAX_BATCH * H * 4, &ok);
     c->mbuf = dalloc(c, (size_t)3 * H * 4, &ok);
     c->ctl = dalloc(c, 16 * 4, &ok);
     c->vt = dalloc(c, (E_MAX_K + 2) * 4, &ok);
@@ -229,8 +240,8 @@ static int check_tokens(const pinfer_ctx *c, const int32_t *tokens, int n) {
 
 /* engine/src/forward.c:154-165 with logits of the last token only. */
 static int eval_chunks(pinfer_ctx *c, const int32_t *tokens, int n, int want_logits) {
-    for (int t0 = 0; t0 < n; t0 += E_MAX_BATCH) {
-        const int nb = n - t0 < E_MAX_BATCH ? n - t0 : E_MAX_BATCH;
+    for (int t0 = 0; t0 < n; t0 += c->chunk) {
+        const int nb = n - t0 < c->chunk ? n - t0 : c->chunk;
         if (nmx_upload(c->dev, c->tok, tokens + t0, (size_t)nb * 4)) return PINFER_E_ARG;
         int rc = e_set_pos(c, c->n_past);
         if (rc == PINFER_OK) rc = e_forward(c, c->tok, nb, 0, 0);

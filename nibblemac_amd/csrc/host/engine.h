@@ -10,7 +10,9 @@
 #include "nmx.h"
 #include "pinfer.h"
 
-#define E_MAX_BATCH 64   /* rows per forward chunk (the reference's PF_MAX_BATCH) */
+#define E_MAX_BATCH 64   /* committed rows queued for the MTP pass */
+#define E_CHUNK NMX_CHUNK_ROWS /* most rows of a prompt per forward pass */
+#define E_SCORE_BYTES ((size_t)512 << 20) /* attention scores workspace above 64 rows */
 #define E_MAX_K PINFER_SPEC_MAX_K
 #define E_MAX_ALLOCS 96  /* device allocations per context besides the weight blob */
 
@@ -36,10 +38,10 @@ typedef struct {
     const float *q_norm, *k_norm;
 } e_layer;
 
-/* one set of per-row scratch buffers (E_MAX_BATCH rows) */
+/* one set of per-row scratch buffers (pinfer_ctx.chunk rows) */
 typedef struct {
     float *x, *x2, *xn, *out, *ta, *tb, *tc, *to, *conv, *ba, *aa, *beta, *decay, *cat, *emb;
-    float *sc; /* attention scores [B][n_heads][max_ctx] */
+    float *sc; /* attention scores [score_rows][n_heads][max_ctx] */
     nmx_a8 a_h;        /* A8 of width hidden */
     nmx_a8 a_w;        /* A8 of the wide inputs: vd, n_heads * head_dim, 2 * hidden */
     nmx_a8 a_f;        /* A8 of width ffn */
@@ -105,6 +107,9 @@ struct pinfer_ctx {
     float rms_eps, rope_theta;
     int n_lin, n_full, has_mtp;
     int max_ctx;
+    int chunk;                /* rows of a prompt per forward pass: E_CHUNK, or 64 where the
+                               * DeltaNet chunk kernels do not take the model's shape */
+    int score_rows;
 
     /* weights: the .pq data section uploaded as one block */
     void *blob;
@@ -130,13 +135,13 @@ struct pinfer_ctx {
     float *rope_cos, *rope_sin;
 
     e_scratch s;
-    float *hbuf;              /* [E_MAX_BATCH][H] final-normed rows kept for the MTP pass */
+    float *hbuf;              /* [chunk][H] final-normed rows kept for the MTP pass */
     float *pbuf;              /* [E_MAX_BATCH][H] committed rows waiting for the MTP pass
                                * (plain steps, n-gram rounds) */
     float *mbuf;              /* [3][H]: MTP hidden of the current draft + chain ping-pong */
     int32_t *ctl;             /* [16] control block (see nmx.h) */
     int32_t *vt;              /* [E_MAX_K + 2] verify tokens */
-    int32_t *tok;             /* [E_MAX_BATCH] tokens of an eager forward */
+    int32_t *tok;             /* [chunk] tokens of an eager forward */
     int32_t *hout;            /* [2 + E_MAX_BATCH] head output */
     int32_t *hout2;           /* [2 + 1] MTP head output */
     int32_t *dcopy;           /* [E_MAX_K + 2] the verify head's copy of the drafts */

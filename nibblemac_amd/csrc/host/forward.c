@@ -64,8 +64,16 @@ static void resid_done(e_resid *r) {
 static int proj_in(pinfer_ctx *c, int count, const void *const *W, const int *R, float *const *Y,
                    int n, const nmx_norm_in *in) {
     e_scratch *s = &c->s;
-    if (in) CK(nmx_q4k_matmul_norm(c->dev, count, W, R, Y, R, c->H, n, in, s->a_h));
-    else CK(nmx_q4k_matmul_multi(c->dev, count, W, R, Y, R, c->H, n, s->a_h.q, s->a_h.d, s->a_h.fs));
+    if (in) CK(nmx_q4k_matmul_norm_chunk(c->dev, count, W, R, Y, R, c->H, n, in, s->a_h));
+    else CK(nmx_q4k_matmul_chunk(c->dev, count, W, R, Y, R, c->H, n, s->a_h.q, s->a_h.d, s->a_h.fs));
+    return PINFER_OK;
+}
+
+/* Y [n][rows] = W a for one matrix and the A8 rows a (more than 64 in a prompt's chunk) */
+static int proj(pinfer_ctx *c, const e_mat *W, int rows, int cols, int n, nmx_a8 a, float *Y) {
+    const void *w[1] = {W->w};
+    float *y[1] = {Y};
+    CK(nmx_q4k_matmul_chunk(c->dev, 1, w, &rows, y, &rows, cols, n, a.q, a.d, a.fs));
     return PINFER_OK;
 }
 
@@ -85,10 +93,8 @@ static int attn_block(pinfer_ctx *c, const e_layer *L, int n, void *kc, void *vc
     nmx_attn_args a = {n, c->n_heads, c->n_kv, hd, c->rot, c->max_ctx, s->ta, s->tb, s->tc,
                        L->q_norm, L->k_norm, c->rms_eps, 1.0f / sqrtf((float)hd), c->rope_cos,
                        c->rope_sin, kc, vc, c->ctl, pos_off, s->to, s->a_w, s->sc, c->kv_dtype};
-    CK(nmx_attn_fused(D, &a)); /* prep + scores in one launch, then P.V */
-    CK(nmx_q4k_matmul(D, L->o.w, H, c->n_heads * hd, n, s->a_w.q, s->a_w.d, s->a_w.fs, s->out,
-                      H, NULL));
-    return PINFER_OK;
+    CK(nmx_attn_fused_chunk(D, &a, c->score_rows)); /* prep + scores in one launch, then P.V */
+    return proj(c, &L->o, H, c->n_heads * hd, n, s->a_w, s->out);
 }
 
 /* post norm + SwiGLU MLP (engine/src/forward.c:49-58): x += mix out; xn = norm(x);
@@ -100,13 +106,13 @@ static int mlp_block(pinfer_ctx *c, const e_layer *L, int n, e_resid *r) {
     e_scratch *s = &c->s;
     const int H = c->H, F = c->ffn;
     const nmx_norm_in in = {r->cur, H, s->out, H, r->alt, H, L->post_norm, c->rms_eps};
-    CK(nmx_q4k_swiglu(D, L->gate.w, L->up.w, F, H, n, NULL, NULL, NULL, &in, NULL, s->a_f, s->a_h,
-                      s->ta, s->tb));
+    CK(nmx_q4k_swiglu_chunk(D, L->gate.w, L->up.w, F, H, n, NULL, NULL, NULL, &in, NULL, s->a_f,
+                            s->a_h, s->ta, s->tb));
     float *t = r->cur; /* the sum x + out is the residual stream now */
     r->cur = r->alt;
     r->alt = t;
     r->add = NULL;
-    CK(nmx_q4k_matmul(D, L->down.w, H, F, n, s->a_f.q, s->a_f.d, s->a_f.fs, s->out, H, NULL));
+    TRY(proj(c, &L->down, H, F, n, s->a_f, s->out));
     r->add = s->out;
     return PINFER_OK;
 }
@@ -136,9 +142,8 @@ static int lin_block(pinfer_ctx *c, const e_layer *L, int n, int logged, const n
                       c->cap - 1, 0, c->ctl + 2};
     /* conv + gates, recurrence, gated norm + A8 of o: one launch */
     nmx_lin_mix_args m = {p, a, s->tb, vd, L->lin_norm, c->rms_eps, NULL, 0, s->a_w};
-    CK(nmx_lin_mix(D, &m));
-    CK(nmx_q4k_matmul(D, L->out.w, H, vd, n, s->a_w.q, s->a_w.d, s->a_w.fs, s->out, H, NULL));
-    return PINFER_OK;
+    CK(nmx_lin_mix_chunk(D, &m));
+    return proj(c, &L->out, H, vd, n, s->a_w, s->out);
 }
 
 int e_keys_ok(const pinfer_ctx *c) { return c->H % 256 == 0 && c->H <= 1024; }
@@ -236,8 +241,7 @@ int e_mtp_forward(pinfer_ctx *c, const float *h_dev, int32_t *tok_dev, int n, in
         CK(nmx_embed_norm(D, c->embed.w, c->vocab, tok_dev, n, H, c->rms_eps, c->mtp_norm_emb,
                           s->emb, H, s->cat, 2 * H, a8_emb, h_dev, H, c->mtp_norm_hid, s->cat + H,
                           2 * H, a8_hid));
-        CK(nmx_q4k_matmul(D, c->mtp_fc.w, H, 2 * H, n, s->a_w.q, s->a_w.d, s->a_w.fs, r.cur, H,
-                          NULL));
+        TRY(proj(c, &c->mtp_fc, H, 2 * H, n, s->a_w, r.cur));
     }
     const e_layer *L = &c->mtp;
     const nmx_norm_in in = resid_norm(c, &r, L->in_norm);

@@ -234,9 +234,9 @@ static int zero_mtp_rows(pinfer_ctx *c, int p0, int p1) {
 static int prefill(pinfer_ctx *c, const int32_t *prompt, int n, int use_mtp, int nv) {
     const int base = c->n_past;
     if (use_mtp && c->mtp_rows < base) TRY(zero_mtp_rows(c, c->mtp_rows, base));
-    int32_t next[E_MAX_BATCH];
-    for (int c0 = 0; c0 < n; c0 += E_MAX_BATCH) {
-        const int nb = n - c0 < E_MAX_BATCH ? n - c0 : E_MAX_BATCH, last = c0 + nb == n;
+    int32_t next[E_CHUNK];
+    for (int c0 = 0; c0 < n; c0 += c->chunk) {
+        const int nb = n - c0 < c->chunk ? n - c0 : c->chunk, last = c0 + nb == n;
         CK(nmx_upload(c->dev, c->tok, prompt + c0, (size_t)nb * sizeof(int32_t)));
         TRY(e_set_pos(c, c->n_past));
         TRY(e_forward(c, c->tok, nb, 0, 0));
