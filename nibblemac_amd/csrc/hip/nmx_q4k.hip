@@ -961,6 +961,207 @@ __global__ __launch_bounds__(64 * MM_S) __attribute__((amdgpu_waves_per_eu(2))) 
     if (sb < nsb) superblock(A, sb);
 }
 
+/* The same for more tiles than one round of workgroups holds: a workgroup owns 16 rows and walks over
+ * T vector tiles. Each of its S waves keeps one superblock's codes and scales in registers (its mins
+ * in LDS), so per tile it loads activations only, two tiles ahead, and the tiles follow each other
+ * through the waves like through a pipeline: wave w takes tile t's accumulators from wave w - 1, runs
+ * its 8 blocks, hands them on. More than MN_S superblocks run as rounds of S, the accumulators of
+ * every tile waiting in LDS between rounds. Progress counters in LDS order it: a wave waits for the
+ * wave before it on this tile, and for the wave after it two tiles back (the two hand-over slots);
+ * both are earlier in the order (round, tile, wave), so every wait ends.
+ * Bound: instruction issue, about 220 per 16 x 16 x 256 tile, at some 290 clocks per tile and CU. The
+ * mins stay in LDS, read two blocks ahead, so that three waves of 168 registers fit a SIMD without
+ * spills. Two row groups per wave (half the activation traffic): no faster at 7168 x 1024. us of
+ * this kernel / of q4k_mm_k at 512 vectors: 1024 x 2048 13.9 / 23.8, 1024 x 3584 20.9 / 30.1, 7168 x
+ * 1024 32.5 / 77.8, 8224 x 1024 39.6 / 89.2; at 64: 7168 x 1024 9.5 / 12.8, 8224 x 1024 10.6 / 15.4. */
+constexpr int MN_S = 8;  /* most waves of a workgroup */
+constexpr int MN_T = 32; /* most vector tiles of a workgroup */
+
+struct MnLds { /* dynamic LDS of a launch of S waves: byte offsets */
+    int scl, df, hand, carry, total;
+};
+__host__ __device__ constexpr MnLds mn_lds(int S, int T, bool rounds) {
+    return {S * 256, S * 1280, S * 2304, S * 4352, S * 4352 + (rounds ? T * 1024 : 0)};
+}
+
+__global__ __launch_bounds__(64 * MN_S) __attribute__((amdgpu_waves_per_eu(3))) void q4k_mmn_k(
+    SegTable tab, int cols, int n, int T, const int8_t *__restrict__ q, const float *__restrict__ d,
+    const float *__restrict__ fs) {
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    extern __shared__ __align__(16) uint8_t lds[];
+    __shared__ int prog[MN_S]; /* tiles done by each wave, over all rounds */
+    const int tid = threadIdx.x, lane = tid & 63, S = blockDim.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, c16 = lane & 15, nsb = cols >> 8;
+    const int grp = blockIdx.x; /* 16-row group over all segments */
+    const uint8_t *W = tab.s[0].W;
+    float *Y = tab.s[0].Y;
+    int rows = tab.s[0].rows, ystride = tab.s[0].ystride, grp0 = tab.s[0].wave0;
+#pragma unroll
+    for (int t = 1; t < NMX_MAX_SEGS; t++)
+        if (t < tab.count && grp >= tab.s[t].wave0) {
+            W = tab.s[t].W;
+            Y = tab.s[t].Y;
+            rows = tab.s[t].rows;
+            ystride = tab.s[t].ystride;
+            grp0 = tab.s[t].wave0;
+        }
+    const MnLds L = mn_lds(S, T, nsb > S);
+    uint8_t *raw = lds + w * 256;                   /* the superblock's scale lines, 4 tiles x 64 bytes */
+    float *scl = (float *)(lds + L.scl + w * 1024); /* [block][D s | M m][16 rows] */
+    float2 *df = (float2 *)(lds + L.df + w * 1024); /* (d, fsum) [block][16 vectors] */
+    float4 *hand = (float4 *)(lds + L.hand), *carry = (float4 *)(lds + L.carry);
+    if (tid < MN_S) prog[tid] = 0;
+    __syncthreads();
+    const int row0 = (grp - grp0) * 16, tile0 = row0 >> 2, rtiles = rows >> 2;
+    const int v0 = blockIdx.y * T * 16;
+    const int Tn = (n - v0 + 15) / 16 < T ? (n - v0 + 15) / 16 : T; /* vector tiles here */
+    const uint32_t tb = (uint32_t)nsb * SB_BYTES;
+    const uint8_t *Wb = W + (size_t)tile0 * tb;
+    /* as in q4k_mm_k: the lane's byte offsets, clamped into the matrix and the vectors */
+    auto tile_at = [&](int t) { return (uint32_t)(tile0 + t < rtiles ? t : rtiles - 1 - tile0) * tb; };
+    const uint32_t oc = tile_at(c16 >> 2) + 64 + 16 * (c16 & 3) + 8 * (g & 1);
+    const uint32_t os = tile_at(lane >> 4) + 4 * (lane & 15);
+    const int sh = 4 * (g >> 1);
+    constexpr int BIAS = 0x4b400000; /* the bits of 1.5 * 2^23 */
+    const v4i bias = {BIAS, BIAS, BIAS, BIAS};
+    auto done = [&](int i) {
+        return __hip_atomic_load(&prog[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+
+    for (int r = 0, sb0 = 0; sb0 < nsb; r++, sb0 += S) {
+        const int sb = sb0 + w, last = (nsb - sb0 < S ? nsb - sb0 : S) - 1; /* the round's last wave */
+        if (w > last) break; /* only in the last round; nobody waits for the wave there */
+        const uint8_t *wb = Wb + (size_t)sb * SB_BYTES;
+        const int8_t *qb = q + (size_t)sb * 256 * n;
+        const float *db = d + (size_t)sb * 8 * n, *fb = fs + (size_t)sb * 8 * n;
+        u32x2 c[8];
+        struct Act {
+            u32x2 x[8];
+            float d0, d1, f0, f1;
+        };
+        auto fetch = [&](Act &A, int tt) {
+            const int t = tt < Tn ? tt : Tn - 1, va = v0 + 16 * t + c16, v = va < n ? va : n - 1;
+            const uint32_t od = (uint32_t)(g * n + v), ox = (uint32_t)v * 32 + 8 * g;
+            A.d0 = db[od], A.d1 = db[od + 4 * (uint32_t)n];
+            A.f0 = fb[od], A.f1 = fb[od + 4 * (uint32_t)n];
+#pragma unroll
+            for (int k = 0; k < 8; k++) A.x[k] = *(const u32x2 *)(qb + ox + (uint32_t)(k * n) * 32);
+        };
+        const uint32_t sraw = *(const uint32_t *)(wb + os);
+#pragma unroll
+        for (int k = 0; k < 8; k++) c[k] = *(const u32x2 *)(wb + oc + 64 * k);
+        Act A0, A1;
+        fetch(A0, 0);
+        fetch(A1, 1);
+        /* the scales: lane = row c16, blocks g and g + 4 (exact: 6-bit x 11-bit) */
+        *(uint32_t *)(raw + 4 * lane) = sraw;
+        __builtin_amdgcn_wave_barrier();
+        {
+            const int i = c16 & 3;
+            const uint8_t *p = raw + 64 * (c16 >> 2);
+            const float D = half_bits_to_float(*(const uint16_t *)(p + 2 * i));
+            const float M = half_bits_to_float(*(const uint16_t *)(p + 8 + 2 * i));
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const int k = g + 4 * u, j = 4 * k + i;
+                scl[k * 32 + c16] = D * (float)nmx_get6(p + 16, j);
+                scl[k * 32 + 16 + c16] = M * (float)nmx_get6(p + 40, j);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        float sc[8][4];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float4 s4 = *(const float4 *)(scl + k * 32 + 4 * g);
+            sc[k][0] = s4.x, sc[k][1] = s4.y, sc[k][2] = s4.z, sc[k][3] = s4.w;
+            c[k].x = (c[k].x >> sh) & 0x0f0f0f0fu, c[k].y = (c[k].y >> sh) & 0x0f0f0f0fu;
+        }
+        auto tile = [&](Act &A, int t) {
+            const int idx = r * Tn + t;
+            df[lane] = make_float2(A.d0, A.f0);
+            df[64 + lane] = make_float2(A.d1, A.f1);
+            __builtin_amdgcn_wave_barrier();
+            float2 dv[8]; /* read here: an LDS read takes longer than a block's arithmetic */
+#pragma unroll
+            for (int k = 0; k < 8; k++) dv[k] = df[k * 16 + c16];
+            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (sb > 0) {
+                const int from = w > 0 ? w - 1 : S - 1, need = w > 0 ? idx : idx - Tn;
+                while (done(from) <= need) {
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                const float4 a = w > 0 ? hand[(from * 2 + (idx & 1)) * 64 + lane] : carry[t * 64 + lane];
+                acc[0] = a.x, acc[1] = a.y, acc[2] = a.z, acc[3] = a.w;
+            }
+            /* block k: its chains, behind the dots of block k + 1 and the mins of block k + 2 */
+            v4i dot[2];
+            auto dots = [&](int k) {
+                dot[k & 1] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                    (long)c[k].x | ((long)c[k].y << 32), (long)A.x[k].x | ((long)A.x[k].y << 32), bias,
+                    0, 0, 0);
+            };
+            float4 of[3];
+            of[0] = *(const float4 *)(scl + 16 + 4 * g);
+            of[1] = *(const float4 *)(scl + 32 + 16 + 4 * g);
+            dots(0);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (k < 7) dots(k + 1);
+                if (k < 6) of[(k + 2) % 3] = *(const float4 *)(scl + (k + 2) * 32 + 16 + 4 * g);
+                if (k == 6) fetch(A, t + 2);
+                const float o[4] = {of[k % 3].x, of[k % 3].y, of[k % 3].z, of[k % 3].w};
+                float fd[4], sd[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    sd[j] = sc[k][j] * dv[k].x;
+                    fd[j] = __int_as_float(dot[k & 1][j]) - 12582912.0f;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(fd[j], sd[j], acc[j]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(-o[j], dv[k].y, acc[j]);
+                /* here, not where a later block needs it: instruction selection otherwise sinks the
+                 * chains past the loads and keeps their operands */
+#pragma unroll
+                for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[j]));
+            }
+            const float4 out = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            if (sb + 1 == nsb) {
+                const int row = row0 + 4 * g, v = v0 + 16 * t + c16; /* a whole 4-row tile */
+                if (row < rows && v < n) {
+                    float *y = Y + (size_t)v * ystride + row;
+                    if (((uintptr_t)Y & 15) == 0 && ystride % 4 == 0) {
+                        *(float4 *)y = out;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) y[j] = acc[j];
+                    }
+                }
+            } else if (w < last) {
+                if (idx >= 2)
+                    while (done(w + 1) < idx - 1) {
+                    }
+                hand[(w * 2 + (idx & 1)) * 64 + lane] = out;
+            } else {
+                carry[t * 64 + lane] = out;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            if (lane == 0)
+                __hip_atomic_store(&prog[w], idx + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        };
+        /* whole pairs, so that a wait for one set of loads does not wait for the other */
+        int t = 0;
+        for (; t + 2 <= Tn; t += 2) {
+            tile(A0, t);
+            tile(A1, t + 1);
+        }
+        if (t < Tn) tile(A0, t);
+    }
+}
+
 /* A8 quantization, one 32-lane half-wave per (block b, vector v) unit; unit index = b * n + v,
  * which is the block-major output index (engine/src/kern.h:19-27). Cross-lane max of |x| and
  * the int sum are exact in any order; 127 / amax and amax / 127 are IEEE divides; the code is
@@ -1102,7 +1303,16 @@ int launch_ksplit(nmx_ctx *ctx, const SegTable &tab, int total_rows_groups, int 
     return 0;
 }
 
-/* More than 8 vectors (prefill chunks): the MFMA kernel, its segment table counting 16-row groups. */
+/* More than 8 vectors (prefill chunks): the MFMA kernels, their segment table counting 16-row
+ * groups. q4k_mm_k, a workgroup per tile, while its workgroups are resident at once (two of 4 waves
+ * per CU, by its registers: 512), where a tile's latency decides (us against q4k_mmn_k: 1024 x 2048
+ * at 128 vectors 8.0 against 9.3, 1024 x 3584 9.8 against 12.7); above that its rounds add up, and
+ * q4k_mmn_k shares a row group's weights among the tiles (1024 x 2048 at 256 vectors 13.4 against
+ * 10.5, 7168 x 1024 at 32 8.0 against 7.7). There a row group gets as many workgroups as stay
+ * resident: three of up to 4 waves per CU, one of more (1024 x 3584 at 512 vectors: 256 workgroups
+ * 20.9 us, 320 28.5 us). */
+constexpr int MM_RESIDENT = 512, MN_RESIDENT = 256;
+
 int launch_mm(nmx_ctx *ctx, SegTable tab, int cols, int n, const int8_t *q, const float *d,
               const float *fs) {
     int groups = 0;
@@ -1111,8 +1321,27 @@ int launch_mm(nmx_ctx *ctx, SegTable tab, int cols, int n, const int8_t *q, cons
         groups += (tab.s[s].rows + 15) / 16;
     }
     tab.total_waves = groups;
-    const dim3 grid((unsigned)groups, (unsigned)((n + 15) / 16));
-    q4k_mm_k<<<grid, 64 * MM_S, 0, ctx->stream>>>(tab, cols, n, q, d, fs);
+    const int vtiles = (n + 15) / 16, nsb = cols >> 8;
+    if ((long)groups * vtiles <= MM_RESIDENT) {
+        const dim3 grid((unsigned)groups, (unsigned)vtiles);
+        q4k_mm_k<<<grid, 64 * MM_S, 0, ctx->stream>>>(tab, cols, n, q, d, fs);
+    } else {
+        const int rounds = (nsb + MN_S - 1) / MN_S, S = (nsb + rounds - 1) / rounds;
+        const int resident = S <= 4 ? 3 * MN_RESIDENT : MN_RESIDENT;
+        int parts = groups < resident ? resident / groups : 1;
+        if (parts > vtiles) parts = vtiles;
+        int T = (vtiles + parts - 1) / parts;
+        if (T > MN_T) T = MN_T;
+        static bool ready = false; /* idempotent */
+        if (!ready) {
+            NMX_HIP(ctx, hipFuncSetAttribute((const void *)q4k_mmn_k,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             mn_lds(MN_S, MN_T, true).total));
+            ready = true;
+        }
+        const dim3 grid((unsigned)groups, (unsigned)((vtiles + T - 1) / T));
+        q4k_mmn_k<<<grid, 64 * S, (size_t)mn_lds(S, T, nsb > S).total, ctx->stream>>>(tab, cols, n, T, q, d, fs);
+    }
     NMX_LAUNCHED(ctx, "q4k_mm");
     return 0;
 }
