@@ -16,8 +16,8 @@
  *   - 8 columns per workgroup of 4 waves (two on the kv chains, two on o): one wave per SIMD, 256
  *     workgroups at 16 heads x 128 columns, where lin_mix_k's one workgroup per head left 240 CUs
  *     idle and put two chain waves on each SIMD.
- * 64 tokens, 16 heads x 128 x 128: 39.8 us, 0.58 us per token above the pipeline's fill (lin_mix_k,
- * conv and gated norm included: 97-100 us, 1.45 us per token). */
+ * 64 tokens, 16 heads x 128 x 128: 36.3 us, 500 tokens 210 us, 0.41 us per token (lin_mix_k, conv and
+ * gated norm included: 97-100 us for 64, 1.45 us per token). */
 #include "nmx_internal.h"
 #include "nmx_linc.h"
 #include "nmx_lanes.h"
@@ -101,10 +101,14 @@ __global__ __launch_bounds__(256) void lin_prec_k(nmx_lin_pre_args a) {
         if (u < nb && live) a.out[(size_t)(t0 + u) * a.C + ch] = y[u];
 }
 
-constexpr int RC_TB = 16;  /* tokens per batch: one barrier, one staged batch */
-constexpr int RC_RING = 4; /* batches in LDS: being staged, in the kv chains, two in the o chains */
+/* Tokens run in batches of TB (one barrier, one staged batch each). The o chains end a batch and 15
+ * steps after the kv chains, which restart their operand reads at every batch: batches of 8 for
+ * chunks of up to RC_SHORT tokens, where the end counts (45 tokens 27.5 us, 31.3 in batches of 16; 64
+ * tokens 36.3 and 39.8), of 16 above (500 tokens 210 us, 212 in batches of 8). */
+constexpr int RC_SHORT = 192;
 constexpr int RC_JW = 8;   /* value columns per workgroup */
-constexpr int RC_TOK = RC_TB * RC_RING;
+constexpr int RC_TOK = 64; /* tokens in LDS: a batch being staged, one in the kv chains, those of the
+                            * last 15 steps in the o chains */
 
 /* LDS row stride of a token's keys: 16 lanes reading their keys of 16 consecutive tokens are
  * 4 (mod 64) words apart, so their 16-byte reads cover the banks once */
@@ -126,12 +130,13 @@ __device__ __forceinline__ float from_prev(float v) {
 
 /* KP keys per lane (dk = 16 KP). Waves 0, 1: kv chains of columns 4 w .. 4 w + 3; waves 2, 3: o
  * chains of the same columns, and the staging of every batch. Iteration i: batch i in the kv
- * chains, the steps of batch i - 1 in the o chains (reaching back 15 tokens into batch i - 2),
+ * chains, the steps of batch i - 1 in the o chains (reaching back 15 tokens),
  * batch i + 1 staged. */
-template <int KP>
+template <int KP, int RC_TB>
 __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *__restrict__ raw,
                                                    int raw_stride, float *__restrict__ conv, int C) {
-    constexpr int DK = 16 * KP, ROW = rc_row(DK);
+    constexpr int DK = 16 * KP, ROW = rc_row(DK), RC_RING = RC_TOK / RC_TB;
+    constexpr int RC_LAG = 1 + (15 + RC_TB - 1) / RC_TB; /* batches from the kv chains' end to the o's */
     extern __shared__ __align__(16) float sm[];
     float *sk = sm, *sq = sk + RC_TOK * ROW;          /* [RC_TOK][ROW] */
     float *sv = sq + RC_TOK * ROW, *sdel = sv + RC_TOK * RC_JW; /* [RC_TOK][RC_JW] */
@@ -141,15 +146,6 @@ __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *
     const int n = a.n, heads = a.heads, dv = a.dv, kh = h / a.rep, kd = (heads / a.rep) * DK;
     const int nbat = (n + RC_TB - 1) / RC_TB;
     const bool kvw = wave < 2;
-
-    /* the chunk's last rows are the next conv state (lin_prec_k has read the old one) */
-    if (conv) {
-        const int nth = gridDim.x * gridDim.y * 256;
-        for (int x = (blockIdx.y * gridDim.x + blockIdx.x) * 256 + tid; x < 3 * C; x += nth) {
-            const int r = x / C, c = x - r * C;
-            conv[x] = raw[(size_t)(n - 3 + r) * raw_stride + c];
-        }
-    }
 
     float *Sp = a.S + state_lane(h, j, part >> 2, DK, dv);
     const int SS = state_slot(j, dv), k0 = (part & 3) * (KP / 4);
@@ -192,12 +188,13 @@ __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *
             fq[e] = *(const float4 *)row;
             fk[e] = *(const float4 *)(row + kd);
         }
-        int t = b * RC_TB + x0 / RC_JW; /* 128 threads: 16 tokens x 8 columns */
+        const int xv = x0 % (RC_TB * RC_JW); /* RC_TB tokens x 8 columns */
+        int t = b * RC_TB + xv / RC_JW;
         t = t < n ? t : n - 1;
-        fv = a.qkv[(size_t)t * a.qkv_stride + 2 * kd + h * dv + j0 + x0 % RC_JW];
-        int tg = b * RC_TB + (x0 & 15);
+        fv = a.qkv[(size_t)t * a.qkv_stride + 2 * kd + h * dv + j0 + xv % RC_JW];
+        int tg = b * RC_TB + x0 % RC_TB;
         tg = tg < n ? tg : n - 1;
-        fg = (x0 < 16 ? a.decay : a.beta)[(size_t)tg * heads + h];
+        fg = (x0 < RC_TB ? a.decay : a.beta)[(size_t)tg * heads + h];
     };
     auto stage = [&](int b) {
         const int s0 = (b % RC_RING) * RC_TB;
@@ -207,9 +204,9 @@ __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *
             *(float4 *)(sq + o) = fq[e];
             *(float4 *)(sk + o) = fk[e];
         }
-        sv[s0 * RC_JW + x0] = fv;
-        if (x0 < 16) sdec[s0 + x0] = fg;
-        else if (x0 < 32) sbet[s0 + x0 - 16] = fg;
+        if (x0 < RC_TB * RC_JW) sv[s0 * RC_JW + x0] = fv;
+        if (x0 < RC_TB) sdec[s0 + x0] = fg;
+        else if (x0 < 2 * RC_TB) sbet[s0 + x0 - RC_TB] = fg;
     };
     if (!kvw) {
         request(0);
@@ -217,7 +214,7 @@ __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *
     }
     __syncthreads();
     float acc = 0.0f;
-    for (int i = 0; i < nbat + 2; i++) {
+    for (int i = 0; i < nbat + RC_LAG; i++) {
         if (kvw) {
             if (i < nbat) {
                 const int tn = n - i * RC_TB < RC_TB ? n - i * RC_TB : RC_TB;
@@ -259,24 +256,41 @@ __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *
             }
         } else {
             if (i + 1 < nbat) request(i + 1);
-            const int tau0 = (i - 1) * RC_TB;
             if (i > 0) {
+                const int tau0 = (i - 1) * RC_TB;
+                float k[KP], q[KP], dec, del;
+                auto operands = [&](int u) { /* of step u; outside the chunk some slot's, unused */
+                    const int sl = (tau0 + u - part) & (RC_TOK - 1);
+                    load_keys(k, sk + sl * ROW + part * KP);
+                    load_keys(q, sq + sl * ROW + part * KP);
+                    dec = sdec[sl], del = sdel[sl * RC_JW + jl];
+                };
+                operands(0);
+#pragma unroll
                 for (int u = 0; u < RC_TB; u++) {
-                    const int t = tau0 + u - part, sl = t & (RC_TOK - 1);
+                    const int t = tau0 + u - part;
                     acc = from_prev(acc);
+                    float kc[KP], qc[KP];
+                    const float dc = dec, ec = del;
+#pragma unroll
+                    for (int r = 0; r < KP; r++) kc[r] = k[r], qc[r] = q[r];
+                    if (u + 1 < RC_TB) operands(u + 1);
                     if (t >= 0 && t < n) {
-                        float k[KP], q[KP];
-                        load_keys(k, sk + sl * ROW + part * KP);
-                        load_keys(q, sq + sl * ROW + part * KP);
-                        const float dec = sdec[sl], del = sdel[sl * RC_JW + jl];
 #pragma unroll
                         for (int r = 0; r < KP; r++) {
-                            s[r] = s[r] * dec;
-                            s[r] = s[r] + k[r] * del;
-                            acc = acc + s[r] * q[r];
+                            s[r] = s[r] * dc;
+                            s[r] = s[r] + kc[r] * ec;
+                            acc = acc + s[r] * qc[r];
                         }
                         if (part == 15) a.o[(size_t)t * a.o_stride + h * dv + j] = acc;
                     }
+                }
+            } else if (conv) { /* the chunk's last rows are the next conv state (lin_prec_k has read
+                                * the old one) */
+                const int nth = gridDim.x * gridDim.y * 128;
+                for (int x = (blockIdx.y * gridDim.x + blockIdx.x) * 128 + x0; x < 3 * C; x += nth) {
+                    const int r = x / C, c = x - r * C;
+                    conv[x] = raw[(size_t)(n - 3 + r) * raw_stride + c];
                 }
             }
             if (i + 1 < nbat) stage(i + 1);
@@ -290,26 +304,32 @@ __global__ __launch_bounds__(256) void lin_rulec_k(nmx_lin_args a, const float *
     }
 }
 
-template <int KP>
+template <int KP, int TB>
 int launch_rulec(nmx_ctx *ctx, const nmx_lin_args &a, const float *raw, int raw_stride, float *conv,
                  int C) {
     const size_t lds = (2 * (size_t)RC_TOK * rc_row(16 * KP) + 2 * RC_TOK * RC_JW + 2 * RC_TOK) * 4;
     static bool ready = false; /* idempotent */
     if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)lin_rulec_k<KP>,
+        NMX_HIP(ctx, hipFuncSetAttribute((const void *)lin_rulec_k<KP, TB>,
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         ready = true;
     }
     const dim3 grid((unsigned)a.heads, (unsigned)(a.dv / RC_JW));
-    lin_rulec_k<KP><<<grid, 256, lds, ctx->stream>>>(a, raw, raw_stride, conv, C);
+    lin_rulec_k<KP, TB><<<grid, 256, lds, ctx->stream>>>(a, raw, raw_stride, conv, C);
     NMX_LAUNCHED(ctx, "lin_rulec");
     return 0;
 }
 
+template <int TB>
+int dispatch_tb(nmx_ctx *ctx, const nmx_lin_args &a, const float *raw, int raw_stride, float *conv, int C) {
+    if (a.dk == 64) return launch_rulec<4, TB>(ctx, a, raw, raw_stride, conv, C);
+    if (a.dk == 128) return launch_rulec<8, TB>(ctx, a, raw, raw_stride, conv, C);
+    return launch_rulec<16, TB>(ctx, a, raw, raw_stride, conv, C);
+}
+
 int dispatch(nmx_ctx *ctx, const nmx_lin_args &a, const float *raw, int raw_stride, float *conv, int C) {
-    if (a.dk == 64) return launch_rulec<4>(ctx, a, raw, raw_stride, conv, C);
-    if (a.dk == 128) return launch_rulec<8>(ctx, a, raw, raw_stride, conv, C);
-    return launch_rulec<16>(ctx, a, raw, raw_stride, conv, C);
+    return a.n <= RC_SHORT ? dispatch_tb<8>(ctx, a, raw, raw_stride, conv, C)
+                           : dispatch_tb<16>(ctx, a, raw, raw_stride, conv, C);
 }
 
 } // namespace

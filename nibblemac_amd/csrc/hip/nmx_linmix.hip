@@ -445,7 +445,7 @@ int launch_mix(nmx_ctx *ctx, const LinMix &m, size_t lds) {
 /* Whether the chunk kernels (nmx_linc.hip) take the mixer: more than 8 tokens without a log, and
  * intermediate buffers that pass between the kernels (the fused kernel does without them, so a
  * caller may have left them out) and overlap nothing that a later kernel reads or writes. 64
- * tokens, 16 heads of 128: 5.6 + 39.8 + 4.8 us against 97-100 us for lin_mix_k, whose time per token
+ * tokens, 16 heads of 128: 4.6 + 36.3 + 4.7 us against 97-100 us for lin_mix_k, whose time per token
  * is 1.45 us above about 5 us of setup. */
 bool chunk_ok(const nmx_lin_mix_args &a) {
     const nmx_lin_pre_args &p = a.pre;

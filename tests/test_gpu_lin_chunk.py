@@ -8,6 +8,8 @@ sum takes), 16 and 17 (one batch, one more token), 48, 63, 64 (the ring of 4 bat
 replays, shared key heads, dk 64 to 256, a last column group that is not 16 wide."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -82,3 +84,41 @@ def test_mixer_equals_one_launch(dev, case):
     got = run(dev, c, fused=True)
     for k in want:
         assert_bits_equal(got[k], want[k], k)
+
+
+@pytest.mark.parametrize("case", [
+    # n, heads, rep, dk, dv, keep
+    (193, 2, 1, 256, 64, 3), (192, 4, 2, 128, 32, 0), (209, 2, 1, 64, 64, 0), (512, 2, 2, 128, 32, 0),
+], ids=lambda c: "n%d_h%d_rep%d_dk%d_dv%d_keep%d" % c)
+def test_long_chunk_equals_pieces(dev, case):
+    """nmx_lin_mix_chunk above 64 rows (batches of 8 up to 192 tokens, of 16 above) against passes of
+    64 over the same rows, the states carried from one to the next."""
+    n, heads, rep, dk, dv, keep = case
+    print(f"[case] lin long chunk {case}", flush=True)
+    fn = dev.lib.nmx_lin_mix_chunk
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(LinMixArgs)]
+    c = make_case(dev, np.random.default_rng(n + dk), n, heads, rep, dk, dv, logged=False, keep=keep)
+    h, C, vd = c["host"], c["C"], heads * dv
+
+    def passes(step):
+        d = {k: dev.to_device(h[k]) for k in ("A_log", "dt_bias", "conv_w", "state", "S", "pend", "norm_w")}
+        ys = []
+        for t0 in range(0, n, step):
+            m = min(step, n - t0)
+            x = {k: dev.to_device(h[k][t0:t0 + m]) for k in ("raw", "z", "b", "a")}
+            conv, o, y = (dev.zeros((m, w), np.float32) for w in (C, vd, vd))
+            beta, decay = (dev.zeros((m, heads), np.float32) for _ in range(2))
+            pre = LinPreArgs(m, C, c["K"], dk, c["kd"], p(x["raw"]), C, p(conv), p(d["state"]),
+                             p(d["conv_w"]), None, np.float32(1.0 / np.sqrt(dk)), 1e-6, p(x["b"]),
+                             p(x["a"]), heads, heads, p(d["A_log"]), None, p(d["dt_bias"]), p(beta),
+                             p(decay))
+            rule = LinArgs(m, heads, rep, dk, dv, C, vd, p(conv), p(decay), p(beta), p(d["S"]), p(o),
+                           None, p(d["pend"]), keep if t0 == 0 else 0, 0, None)
+            dev.check(fn(dev.ctx, ctypes.byref(LinMixArgs(pre, rule, p(x["z"]), vd, p(d["norm_w"]), 1e-6,
+                                                          p(y), vd, A8(None, None, None)))))
+            dev.sync()
+            ys.append(y.numpy())
+        return np.concatenate(ys), d["S"].numpy(), d["state"].numpy()
+
+    for got, want, what in zip(passes(512), passes(64), ("y", "state", "conv state")):
+        assert_bits_equal(got, want, what)
