@@ -82,7 +82,7 @@ __device__ __forceinline__ const float *kv_scales(const void *cache, const nmx_a
  * hd a multiple of 64 up to 512. */
 int nmx_attn_chunk(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, float *sc);
 /* Softmax and P.V of a few rows over the scores sc, for caches whose score rows do not fit in LDS. */
-int nmx_attn_long(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, float *sc);
+int nmx_attn_long(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, const float *sc);
 
 /* acc += x[0] + ... + x[n-1] in order, x contiguous in LDS and 16-byte aligned: the terms
  * arrive four per ds_read_b128 with immediate offsets, two sets of 32 taking turns (the next

@@ -140,8 +140,8 @@ __global__ __launch_bounds__(512) void attn_scc_k(Attn a, float *__restrict__ sc
  * interleaved partial sums and the tail in order, w_p = e_p * (1 / sum). A segment's exponentials
  * sit in LDS one partial sum after the other (16-byte chain reads); wave 0 adds a segment while
  * the other waves form the next one's, so a long row costs its chain, np / 4 dependent adds. 512
- * threads with 8 reads in flight each: 26 us for 8 rows of 20000 positions, 11.5 us for 512 rows of
- * 4000 (256 threads with one read each: 57.7 and 16.4 us). */
+ * threads with 8 reads in flight each: 11.5 us for 512 rows of 4000 positions (256 threads with one
+ * read each: 16.4 us). */
 constexpr int SM_T = 512;
 
 __global__ __launch_bounds__(SM_T) void attn_sm_k(Attn a, float *__restrict__ sc) {
@@ -306,22 +306,30 @@ __global__ __launch_bounds__(512) void attn_pvc_k(const float *__restrict__ wts,
     }
 }
 
-/* P.V of a few rows over a long context (steps and verify passes in caches past 8192 positions),
- * on the weights of attn_sm_k: workgroup = (32 dims, head, token), wave 0's lanes the chains, one per
- * dim. The chain, one dependent add per position, bounds it (8.1 clocks a step: 68 us for 20000
- * positions), so everything else runs beside it: waves 1-4 store tile i + 1's products w_p v_p[d] in
- * LDS, one row per dim, while wave 0 adds tile i, and have tile i + 2's values and weights in flight.
- * One token at 20000 positions, binary16 cache: 93 us
- * (attn_sm_k before it 26 us; one kernel that formed the weights twice and stored each tile between
- * two chains: 429 us). */
+/* Softmax and P.V of a few rows in caches past 8192 positions (steps and verify passes): workgroup =
+ * (32 dims, head, token). Each forms its row's max and sum itself (attn_sm_k's steps; the 8 workgroups
+ * of a row run them side by side, and a separate launch would cost a short context 2 us), then wave
+ * 0's lanes run the P.V chains, one per dim. The chain, one dependent add per position, bounds it (8.1
+ * clocks a step: 68 us for 20000 positions), so everything else runs beside it: waves 1-4 store tile
+ * i + 1's products w_p v_p[d] in LDS, one row per dim, while wave 0 adds tile i, and have tile i + 2's
+ * values and scores in flight. One token at 20000 positions, binary16 cache: 130 us (one kernel that
+ * stored each tile between two runs of the chains: 429 us). Up to PL_SHORT positions a row is one pass:
+ * layers of 1 token at 50, 3 at 120, 5 at 900 positions take 34.3, 38.6, 57.9 us (34.8, 39.9, 58.1),
+ * 5 at 1500 63.4 (70.4); 8 tokens, 512 workgroups of five waves, lose 1.5 us there (8 at 300: 55.8,
+ * 54.4) and gain past it. */
 constexpr int PL_P = 256;        /* positions per tile */
 constexpr int PL_D = 32;         /* output dims per workgroup: one A8 block */
 constexpr int PL_RS = PL_P + 4;  /* row stride: 16-byte aligned, 4 words apart modulo 64 banks */
+constexpr int PL_SHORT = 1024;   /* positions up to which a row is one pass without the pipeline */
+constexpr int PS_P = 440;        /* positions per tile there: 11 values per thread, none left over */
 
 template <int KVT>
-__global__ __launch_bounds__(320) void attn_pvl_k(const float *__restrict__ wts, Attn a) {
-    constexpr int F4 = PL_D / 4, PER = PL_P * F4 / 256;
-    __shared__ __align__(16) float vt[2][PL_D * PL_RS];
+__global__ __launch_bounds__(320) void attn_pvl_k(const float *__restrict__ sc, Attn a) {
+    constexpr int F4 = PL_D / 4, PER = PL_P * F4 / 256, T = 320;
+    /* the softmax's two segments, then the two tiles of products */
+    __shared__ __align__(16) float buf[2 * PL_D * PL_RS];
+    static_assert(4 * SM_S4 <= PL_D * PL_RS, "a segment fits in a tile's place");
+    __shared__ float red[8];
     const int hd = a.hd, rep = a.nh / a.nkv, S = (hd / PL_D) * a.nkv, tid = threadIdx.x;
     const int sl = blockIdx.x % S, k = blockIdx.x / S; /* a slice of V to one XCD, as attn_pvc_k */
     const int d0 = (sl % (hd / PL_D)) * PL_D, g = sl / (hd / PL_D);
@@ -329,44 +337,9 @@ __global__ __launch_bounds__(320) void attn_pvl_k(const float *__restrict__ wts,
     const int np = *a.pos + a.pos_off + t + 1, ntile = (np + PL_P - 1) / PL_P;
     const size_t R0 = (size_t)g * a.max_ctx;
     const float *vsc = kv_scales<KVT>(a.vc, a);
-    const float *wr = wts + ((size_t)t * a.nh + h) * a.max_ctx;
-    if (tid >= 64) { /* waves 1-4: 8 lanes to a position */
-        const int f0 = tid - 64, c4 = f0 % F4, r0 = f0 / F4;
-        float4 v[PER];
-        float w[PER];
-        auto fetch = [&](int i) { /* clamped: positions past the row are stored and never added */
-#pragma unroll
-            for (int u = 0; u < PER; u++) {
-                int p = i * PL_P + u * (256 / F4) + r0;
-                p = p < np ? p : np - 1;
-                v[u] = kv_load4<KVT>(a.vc, R0 + p, hd, d0 + 4 * c4, vsc);
-                w[u] = wr[p];
-            }
-        };
-        fetch(0);
-        for (int i = 0; i < ntile; i++) {
-            float *q = vt[i & 1] + 4 * c4 * PL_RS + r0;
-#pragma unroll
-            for (int u = 0; u < PER; u++) {
-                float *x = q + u * (256 / F4);
-                x[0] = w[u] * v[u].x;
-                x[PL_RS] = w[u] * v[u].y;
-                x[2 * PL_RS] = w[u] * v[u].z;
-                x[3 * PL_RS] = w[u] * v[u].w;
-            }
-            fetch(i + 1);
-            __syncthreads(); /* tile i stored; tile i - 1 added */
-        }
-        return;
-    }
+    const float *row = sc + ((size_t)t * a.nh + h) * a.max_ctx;
     const float gate = tid < PL_D ? a.q[((size_t)t * a.nh + h) * 2 * hd + hd + d0 + tid] : 0.0f;
-    float o = 0.0f;
-    for (int i = 0; i < ntile; i++) {
-        __syncthreads();
-        const int rows = np - i * PL_P < PL_P ? np - i * PL_P : PL_P;
-        if (tid < PL_D) o = pv_chain4(o, vt[i & 1] + tid * PL_RS, rows);
-    }
-    if (tid < PL_D) {
+    auto finish = [&](float o) { /* lanes tid < PL_D */
         o = o * nmx_sigmoid(gate);
         const int col = h * hd + d0 + tid;
         a.o[(size_t)t * a.nh * hd + col] = o;
@@ -374,7 +347,159 @@ __global__ __launch_bounds__(320) void attn_pvl_k(const float *__restrict__ wts,
             const size_t u = (size_t)(col >> 5) * a.an + t;
             nmx_a8_store(o, a.aq + u * 32, a.ad + u, a.afs + u);
         }
+    };
+    if (np <= PL_SHORT) { /* uniform: the whole workgroup */
+        /* the exponentials in LDS, one partial sum after the other; the first PS_P positions' values
+         * requested at entry, every thread's products stored, then the chains */
+        constexpr int S4 = PL_SHORT / 4 + 4, RS = PS_P + 4, PSR = PS_P * F4 / T;
+        static_assert(PS_P * F4 % T == 0 && 4 * S4 + PL_D * RS <= 2 * PL_D * PL_RS, "fits in the tiles' place");
+        float *e = buf, *vt = buf + 4 * S4;
+        float4 v[PSR];
+        auto values = [&](int base, int rows) {
+#pragma unroll
+            for (int u = 0; u < PSR; u++) { /* clamped, and whole sweeps of the threads left out */
+                if (u * T >= rows * F4) break;
+                const int f = u * T + tid, r = f / F4 < rows ? f / F4 : rows - 1;
+                v[u] = kv_load4<KVT>(a.vc, R0 + base + r, hd, d0 + 4 * (f % F4), vsc);
+            }
+        };
+        int rows = np < PS_P ? np : PS_P;
+        float x[(PL_SHORT + T - 1) / T], mx = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < (PL_SHORT + T - 1) / T; u++)
+            if (u * T + tid < np) x[u] = row[u * T + tid];
+        values(0, rows);
+#pragma unroll
+        for (int u = 0; u < (PL_SHORT + T - 1) / T; u++)
+            if (u * T + tid < np) mx = fmaxf(mx, x[u]);
+        mx = nmx_max_f32_wave(mx);
+        if ((tid & 63) == 0) red[tid >> 6] = mx;
+        __syncthreads();
+        mx = red[0];
+#pragma unroll
+        for (int u = 1; u < T / 64; u++) mx = fmaxf(mx, red[u]);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < (PL_SHORT + T - 1) / T; u++) {
+            const int p = u * T + tid;
+            if (p < np) e[(p & 3) * S4 + (p >> 2)] = nmx_expf_cephes(x[u] - mx);
+        }
+        __syncthreads();
+        if (tid < 4) {
+            red[tid] = pv_chain4(0.0f, e + tid * S4, np >> 2);
+        } else if (tid == 4) {
+            float tl = 0.0f;
+            for (int p = np & ~3; p < np; p++) tl = tl + e[(p & 3) * S4 + (p >> 2)];
+            red[4] = tl;
+        }
+        __syncthreads();
+        const float inv = 1.0f / (((red[0] + red[1]) + (red[2] + red[3])) + red[4]);
+        float o = 0.0f;
+        for (int base = 0; base < np; base += PS_P) {
+#pragma unroll
+            for (int u = 0; u < PSR; u++) {
+                if (u * T >= rows * F4) break;
+                const int f = u * T + tid, r = f / F4, p = base + r < np ? base + r : np - 1;
+                float *y = vt + 4 * (f % F4) * RS + r; /* past the rows: stored, never added */
+                const float w = e[(p & 3) * S4 + (p >> 2)] * inv;
+                y[0] = w * v[u].x;
+                y[RS] = w * v[u].y;
+                y[2 * RS] = w * v[u].z;
+                y[3 * RS] = w * v[u].w;
+            }
+            const int next = base + PS_P, nrows = np - next < PS_P ? np - next : PS_P;
+            if (next < np) values(next, nrows);
+            __syncthreads();
+            if (tid < PL_D) o = pv_chain4(o, vt + tid * RS, rows);
+            __syncthreads();
+            rows = nrows;
+        }
+        if (tid < PL_D) finish(o);
+        return;
     }
+    /* waves 1-4: 8 lanes to a position; the first tile's values requested before the softmax */
+    const int f0 = tid >= 64 ? tid - 64 : 0, c4 = f0 % F4, r0 = f0 / F4;
+    float4 v[PER];
+    float x[PER];
+    auto fetch = [&](int i) { /* clamped: positions past the row are stored and never added */
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            int p = i * PL_P + u * (256 / F4) + r0;
+            p = p < np ? p : np - 1;
+            v[u] = kv_load4<KVT>(a.vc, R0 + p, hd, d0 + 4 * c4, vsc);
+            x[u] = row[p];
+        }
+    };
+    fetch(0);
+    /* f(i, row[i]) for i = i0, i0 + step, .. < end, 8 reads in flight */
+    auto sweep = [&](int i0, int step, int end, auto f) {
+        for (int i = i0; i < end; i += 8 * step) {
+            float y[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) y[u] = row[i + u * step < end ? i + u * step : end - 1];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (i + u * step < end) f(i + u * step, y[u]);
+        }
+    };
+    float mx = -INFINITY;
+    sweep(tid, T, np, [&](int, float y) { mx = fmaxf(mx, y); });
+    mx = nmx_max_f32_wave(mx);
+    if ((tid & 63) == 0) red[tid >> 6] = mx;
+    __syncthreads();
+    mx = red[0];
+#pragma unroll
+    for (int u = 1; u < T / 64; u++) mx = fmaxf(mx, red[u]);
+    auto exps = [&](int s0, float *dst, int i0, int step) {
+        sweep(s0 + i0, step, np - s0 < SM_SEG ? np : s0 + SM_SEG, [&](int p, float y) {
+            dst[(p & 3) * SM_S4 + ((p - s0) >> 2)] = nmx_expf_cephes(y - mx);
+        });
+    };
+    exps(0, buf, tid, T);
+    __syncthreads();
+    const int q4 = np & ~3; /* positions in whole quads */
+    float chain = 0.0f;     /* lane l < 4: partial sum l; lane 4: the tail */
+    for (int s0 = 0, s = 0; s0 < np; s0 += SM_SEG, s ^= 1) {
+        float *seg = buf + s * PL_D * PL_RS;
+        if (tid < 5) {
+            const int full = q4 - s0 < SM_SEG ? q4 - s0 : SM_SEG;
+            if (tid < 4) chain = pv_chain4(chain, seg + tid * SM_S4, full >> 2);
+            else
+                for (int i = full; i < SM_SEG && s0 + i < np; i++)
+                    chain = chain + seg[(i & 3) * SM_S4 + (i >> 2)];
+        } else if (tid >= 64 && s0 + SM_SEG < np) {
+            exps(s0 + SM_SEG, buf + (s ^ 1) * PL_D * PL_RS, tid - 64, T - 64);
+        }
+        __syncthreads();
+    }
+    if (tid < 5) red[tid] = chain;
+    __syncthreads();
+    const float inv = 1.0f / (((red[0] + red[1]) + (red[2] + red[3])) + red[4]);
+
+    if (tid >= 64) {
+        for (int i = 0; i < ntile; i++) {
+            float *q = buf + (i & 1) * PL_D * PL_RS + 4 * c4 * PL_RS + r0;
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                float *y = q + u * (256 / F4);
+                const float w = nmx_expf_cephes(x[u] - mx) * inv;
+                y[0] = w * v[u].x;
+                y[PL_RS] = w * v[u].y;
+                y[2 * PL_RS] = w * v[u].z;
+                y[3 * PL_RS] = w * v[u].w;
+            }
+            fetch(i + 1);
+            __syncthreads(); /* tile i stored; tile i - 1 added */
+        }
+        return;
+    }
+    float o = 0.0f;
+    for (int i = 0; i < ntile; i++) {
+        __syncthreads();
+        const int rows = np - i * PL_P < PL_P ? np - i * PL_P : PL_P;
+        if (tid < PL_D) o = pv_chain4(o, buf + (i & 1) * PL_D * PL_RS + tid * PL_RS, rows);
+    }
+    if (tid < PL_D) finish(o);
 }
 
 template <int KVT>
@@ -402,9 +527,7 @@ int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
 
 } // namespace
 
-int nmx_attn_long(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, float *sc) {
-    attn_sm_k<<<dim3((unsigned)a.nh, (unsigned)a.n), SM_T, 0, ctx->stream>>>(a, sc);
-    NMX_LAUNCHED(ctx, "attn_sm");
+int nmx_attn_long(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, const float *sc) {
     const unsigned pg = (unsigned)((a.hd / PL_D) * a.nh * a.n);
     if (kv_dtype == KV_F16) attn_pvl_k<KV_F16><<<pg, 320, 0, ctx->stream>>>(sc, a);
     else if (kv_dtype == KV_I8) attn_pvl_k<KV_I8><<<pg, 320, 0, ctx->stream>>>(sc, a);

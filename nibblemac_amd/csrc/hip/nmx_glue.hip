@@ -1505,7 +1505,7 @@ int launch_attn(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
 
 template <int KVT>
 int launch_pv(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
-    /* score rows past the LDS go through memory as softmax weights */
+    /* score rows too long for the LDS */
     if (p->max_ctx > PV_ATT_MAX) return nmx_attn_long(ctx, a, KVT, p->scores);
     const unsigned pgrid = (unsigned)((p->hd / PV_DS) * p->nh * p->n);
     const size_t plds = ((size_t)4 * cm_stride(p->max_ctx) + 4 + (size_t)PV_DS * PV_RS) * 4;
