@@ -6,12 +6,23 @@
  * 16-lane rows, one swizzle across them; max and integer sums are exact in any order.
  * nmx_quad_chain: a left-to-right fp32 sum over a quad of lanes, lane c holding the c-th
  * quarter of the terms; the running sum moves to the next lane by a DPP broadcast of lane c
- * (quad_perm [c, c, c, c]), so the adds are one sequential chain. */
+ * (quad_perm [c, c, c, c]), so the adds are one sequential chain. nmx_lds_wave_sync: between
+ * LDS writes of a wave's lanes and other lanes' accesses to the same words. */
 #ifndef NMX_LANES_H
 #define NMX_LANES_H
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+
+/* Orders the LDS accesses of a wave's lanes before it with those after it. A wave's LDS operations
+ * execute in order, so no instruction comes of it; __builtin_amdgcn_wave_barrier alone constrains
+ * scheduling and not memory, and the compiler may move a load of one type over a store of another
+ * across it. */
+__device__ __forceinline__ void nmx_lds_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
 
 template <int CTRL>
 __device__ __forceinline__ int nmx_dpp(int v) {

@@ -870,16 +870,19 @@ __global__ __launch_bounds__(64 * MM_S) __attribute__((amdgpu_waves_per_eu(2))) 
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 
     auto superblock = [&](Buf &B, int sb) {
+        nmx_lds_wave_sync(); /* the wave's reads of its last superblock */
         /* the scales: lane = row c16, blocks g and g + 4 (exact: 6-bit x 11-bit) */
         *(uint32_t *)(raw + 4 * lane) = B.s;
         df[lane] = make_float2(B.d0, B.f0);
         df[64 + lane] = make_float2(B.d1, B.f1);
-        __builtin_amdgcn_wave_barrier();
+        nmx_lds_wave_sync();
         {
             const int i = c16 & 3;
             const uint8_t *p = raw + 64 * (c16 >> 2);
-            const float D = half_bits_to_float(*(const uint16_t *)(p + 2 * i));
-            const float M = half_bits_to_float(*(const uint16_t *)(p + 8 + 2 * i));
+            uint16_t Db, Mb; /* of 32-bit stores */
+            __builtin_memcpy(&Db, p + 2 * i, 2);
+            __builtin_memcpy(&Mb, p + 8 + 2 * i, 2);
+            const float D = half_bits_to_float(Db), M = half_bits_to_float(Mb);
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 const int k = g + 4 * u, j = 4 * k + i;
@@ -887,7 +890,7 @@ __global__ __launch_bounds__(64 * MM_S) __attribute__((amdgpu_waves_per_eu(2))) 
                 scl[k * 32 + 16 + c16] = M * (float)nmx_get6(p + 40, j);
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        nmx_lds_wave_sync();
         float fd[8][4], sd[8][4];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -1055,14 +1058,17 @@ __global__ __launch_bounds__(64 * MN_S) __attribute__((amdgpu_waves_per_eu(3))) 
         Act A0, A1;
         fetch(A0, 0);
         fetch(A1, 1);
+        nmx_lds_wave_sync(); /* the wave's reads of its last superblock */
         /* the scales: lane = row c16, blocks g and g + 4 (exact: 6-bit x 11-bit) */
         *(uint32_t *)(raw + 4 * lane) = sraw;
-        __builtin_amdgcn_wave_barrier();
+        nmx_lds_wave_sync();
         {
             const int i = c16 & 3;
             const uint8_t *p = raw + 64 * (c16 >> 2);
-            const float D = half_bits_to_float(*(const uint16_t *)(p + 2 * i));
-            const float M = half_bits_to_float(*(const uint16_t *)(p + 8 + 2 * i));
+            uint16_t Db, Mb; /* of 32-bit stores */
+            __builtin_memcpy(&Db, p + 2 * i, 2);
+            __builtin_memcpy(&Mb, p + 8 + 2 * i, 2);
+            const float D = half_bits_to_float(Db), M = half_bits_to_float(Mb);
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 const int k = g + 4 * u, j = 4 * k + i;
@@ -1070,7 +1076,7 @@ __global__ __launch_bounds__(64 * MN_S) __attribute__((amdgpu_waves_per_eu(3))) 
                 scl[k * 32 + 16 + c16] = M * (float)nmx_get6(p + 40, j);
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        nmx_lds_wave_sync();
         float sc[8][4];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -1080,9 +1086,10 @@ __global__ __launch_bounds__(64 * MN_S) __attribute__((amdgpu_waves_per_eu(3))) 
         }
         auto tile = [&](Act &A, int t) {
             const int idx = r * Tn + t;
+            nmx_lds_wave_sync(); /* the wave's reads of its last tile */
             df[lane] = make_float2(A.d0, A.f0);
             df[64 + lane] = make_float2(A.d1, A.f1);
-            __builtin_amdgcn_wave_barrier();
+            nmx_lds_wave_sync();
             float2 dv[8]; /* read here: an LDS read takes longer than a block's arithmetic */
 #pragma unroll
             for (int k = 0; k < 8; k++) dv[k] = df[k * 16 + c16];
@@ -1141,9 +1148,12 @@ __global__ __launch_bounds__(64 * MN_S) __attribute__((amdgpu_waves_per_eu(3))) 
                     }
                 }
             } else if (w < last) {
-                if (idx >= 2)
+                if (idx >= 2) {
                     while (done(w + 1) < idx - 1) {
                     }
+                    /* the next wave's read of the slot, before the store into it */
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+                }
                 hand[(w * 2 + (idx & 1)) * 64 + lane] = out;
             } else {
                 carry[t * 64 + lane] = out;
