@@ -299,14 +299,14 @@ int nmx_lin_post(nmx_ctx *ctx, const float *o, int o_stride, const float *z, int
                  const float *w, int n, int heads, int dv, float eps, float *y, int y_stride,
                  nmx_a8 a8);
 
-/* The Gated DeltaNet mixer between in_proj and out_proj in one launch (engine/src/
- * forward_lin.c:36-81, 94-133): nmx_lin_pre for the q / k / v channels and gates of each value
- * head, nmx_lin_rule and nmx_lin_post (gated RMSNorm of o with z and norm_w, output y and / or
- * its A8), with identical results; the conv outputs, gates and o stay on chip. pre.out,
- * pre.beta, pre.decay, rule.qkv, rule.decay, rule.beta and rule.o are only used (and then
- * must be valid buffers) when the shape is outside the fused kernel's limits and the three
- * kernels run instead, and by the chunk kernels that take more than 8 tokens without a log
- * when all of them are given and overlap no other argument. */
+/* The Gated DeltaNet mixer between in_proj and out_proj (engine/src/forward_lin.c:36-81,
+ * 94-133): nmx_lin_pre for the q / k / v channels and gates of each value head, nmx_lin_rule and
+ * nmx_lin_post (gated RMSNorm of o with z and norm_w, output y and / or its A8), with identical
+ * results. One launch in the fused kernel's shapes, whose conv outputs, gates and o stay on chip;
+ * there more than 8 tokens without a log, outside a capture, run as three launches over the
+ * context's own workspace. pre.out, pre.beta, pre.decay, rule.qkv, rule.decay, rule.beta and rule.o
+ * are only used (and then must be valid buffers) when the shape is outside the fused kernel's
+ * limits and the separate kernels run instead. */
 typedef struct {
     nmx_lin_pre_args pre;
     nmx_lin_args rule;
@@ -428,10 +428,12 @@ int nmx_attn_fused(nmx_ctx *ctx, const nmx_attn_args *p);
  * the suffix in everything else (arguments, layouts, results bit for bit: no result depends on the
  * rows it shares a launch with). No counterpart in the reference, whose chunks have at most 64
  * rows; a longer chunk fills the device and spreads a layer's launches over more tokens.
- * nmx_q4k_matmul_chunk is nmx_q4k_matmul_multi. nmx_lin_mix_chunk: above 64 rows only without a
- * log, in the shapes of nmx_lin_chunk_ok (1 if they take it; host only) and with every intermediate
- * buffer given. nmx_attn_fused_chunk: the scores workspace holds score_rows rows, [score_rows][nh]
- * [max_ctx] floats. */
+ * nmx_q4k_matmul_chunk is nmx_q4k_matmul_multi. nmx_lin_mix_chunk writes the intermediate buffers
+ * (pre.out, pre.beta, pre.decay, rule.o; rule.qkv, rule.decay and rule.beta are the first three) when
+ * all are given, of n rows each, and more than 8 tokens run without a log; above 64 rows it refuses
+ * anything else and shapes outside nmx_lin_chunk_ok (1 if they are inside; host only).
+ * nmx_attn_fused_chunk: the scores workspace holds score_rows rows, [score_rows][nh][max_ctx]
+ * floats. */
 #define NMX_CHUNK_ROWS 512
 int nmx_q4k_matmul_chunk(nmx_ctx *ctx, int count, const void *const *W, const int *rows,
                          float *const *Y, const int *y_stride, int cols, int n, const int8_t *q,

@@ -16,7 +16,13 @@ struct nmx_ctx {
     char name[256];
     char err[1024];
     int capturing;
+    /* nmx_lin_mix's intermediates of more than 8 tokens (NMX_MIX_WS bytes; NULL: it does without).
+     * Only eager launches on the stream use it: a graph may be launched on another context. */
+    float *mix_ws;
 };
+
+/* 64 tokens of 65536 floats: the conv outputs, o and gates of 64 heads of 128 x 128 */
+constexpr size_t NMX_MIX_WS = (size_t)16 << 20;
 
 struct nmx_event {
     hipEvent_t ev;

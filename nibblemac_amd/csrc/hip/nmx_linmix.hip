@@ -442,11 +442,11 @@ int launch_mix(nmx_ctx *ctx, const LinMix &m, size_t lds) {
     return 0;
 }
 
-/* Whether the chunk kernels (nmx_linc.hip) take the mixer: more than 8 tokens without a log, and
- * intermediate buffers that pass between the kernels (the fused kernel does without them, so a
- * caller may have left them out) and overlap nothing that a later kernel reads or writes. 64
- * tokens, 16 heads of 128: 4.6 + 36.3 + 4.7 us against 97-100 us for lin_mix_k, whose time per token
- * is 1.45 us above about 5 us of setup. */
+/* Whether the chunk kernels (nmx_linc.hip) take the mixer with these intermediate buffers: more
+ * than 8 tokens without a log, and buffers that overlap nothing that a later kernel reads or writes.
+ * They are the caller's where the caller gave them to be written (nmx_lin_mix_chunk, and the shapes
+ * outside the fused kernel), else the context's. 64 tokens, 16 heads of 128: 4.6 + 36.3 + 4.7 us
+ * against 97-100 us for lin_mix_k, whose time per token is 1.45 us above about 5 us of setup. */
 bool chunk_ok(const nmx_lin_mix_args &a) {
     const nmx_lin_pre_args &p = a.pre;
     const nmx_lin_args &r = a.rule;
@@ -484,17 +484,24 @@ bool chunk_ok(const nmx_lin_mix_args &a) {
     return true;
 }
 
+int mix_chunk(nmx_ctx *ctx, const nmx_lin_mix_args &a) {
+    const nmx_lin_args &r = a.rule;
+    if (nmx_lin_mixc(ctx, a.pre, r)) return -1;
+    return nmx_lin_post(ctx, r.o, r.o_stride, a.z, a.z_stride, a.norm_w, r.n, r.heads, r.dv, a.eps,
+                        a.y, a.y_stride, a.a8);
+}
+
 } // namespace
 
 extern "C" {
 
-static int lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a, int nmax) {
+static int lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a, bool chunk) {
     if (!ctx) return -1;
     if (!a) return nmx_fail(ctx, "nmx_lin_mix: NULL args");
     const nmx_lin_pre_args &p = a->pre;
     const nmx_lin_args &r = a->rule;
     const int n = p.n, dk = p.dk, dv = r.dv;
-    if (n < 1 || n > nmax || n != r.n || dk != r.dk || p.heads != r.heads || !a->z || !a->norm_w ||
+    if (n < 1 || n > (chunk ? NMX_CHUNK_ROWS : 64) || n != r.n || dk != r.dk || p.heads != r.heads || !a->z || !a->norm_w ||
         a->z_stride < r.heads * dv || (a->y && a->y_stride < r.heads * dv) || dv % 32 ||
         p.kd != (r.heads / r.rep) * dk || p.C != 2 * p.kd + r.heads * dv)
         return nmx_fail(ctx, "nmx_lin_mix: inconsistent arguments");
@@ -511,12 +518,28 @@ static int lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a, int nmax) {
     const bool fused = r.rep == 1 && (dk == 64 || dk == 128) && 4 * dv <= MIX_MAX_THREADS &&
                        dk <= dv && 2 * dk + dv <= 4 * dv - 64 && lds <= MIX_LDS && vec_ok &&
                        !(r.log0 && !r.log);
-    if (chunk_ok(*a)) { /* the chunk kernels, through the structs' intermediate buffers */
-        if (nmx_lin_mixc(ctx, p, r)) return -1;
-        return nmx_lin_post(ctx, r.o, r.o_stride, a->z, a->z_stride, a->norm_w, n, r.heads, dv,
-                            a->eps, a->y, a->y_stride, a->a8);
+    if (chunk) { /* the caller gave the intermediate buffers to write */
+        if (chunk_ok(*a)) return mix_chunk(ctx, *a);
+        if (n > 64) return nmx_fail(ctx, "nmx_lin_mix_chunk: n=%d outside the chunk kernels' limits", n);
     }
-    if (n > 64) return nmx_fail(ctx, "nmx_lin_mix_chunk: n=%d outside the chunk kernels' limits", n);
+    if (fused) { /* the structs' buffers stay untouched; not under capture (see nmx_ctx) */
+        const size_t row = (size_t)p.C + (size_t)r.heads * dv + 2 * (size_t)r.heads;
+        if (n > 8 && ctx->mix_ws && !ctx->capturing && (size_t)n * row * 4 <= NMX_MIX_WS) {
+            nmx_lin_mix_args w = *a;
+            w.rule.o = ctx->mix_ws;
+            w.rule.o_stride = r.heads * dv;
+            w.pre.out = w.rule.o + (size_t)n * r.heads * dv;
+            w.pre.beta = w.pre.out + (size_t)n * p.C;
+            w.pre.decay = w.pre.beta + (size_t)n * r.heads;
+            w.rule.qkv = w.pre.out;
+            w.rule.qkv_stride = p.C;
+            w.rule.beta = w.pre.beta;
+            w.rule.decay = w.pre.decay;
+            if (chunk_ok(w)) return mix_chunk(ctx, w);
+        }
+    } else if (chunk_ok(*a)) {
+        return mix_chunk(ctx, *a);
+    }
     if (!fused) { /* the separate kernels, through the intermediate buffers of the structs */
         if (nmx_lin_pre(ctx, &p) || nmx_lin_rule(ctx, &r)) return -1;
         return nmx_lin_post(ctx, r.o, r.o_stride, a->z, a->z_stride, a->norm_w, n, r.heads, dv,
@@ -533,10 +556,10 @@ static int lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a, int nmax) {
     return dk == 64 ? launch_mix<16>(ctx, m, lds) : launch_mix<32>(ctx, m, lds);
 }
 
-int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) { return lin_mix(ctx, a, 64); }
+int nmx_lin_mix(nmx_ctx *ctx, const nmx_lin_mix_args *a) { return lin_mix(ctx, a, false); }
 
 int nmx_lin_mix_chunk(nmx_ctx *ctx, const nmx_lin_mix_args *a) {
-    return lin_mix(ctx, a, NMX_CHUNK_ROWS);
+    return lin_mix(ctx, a, true);
 }
 
 int nmx_lin_chunk_ok(int dk, int dv, int conv_k, int heads) {

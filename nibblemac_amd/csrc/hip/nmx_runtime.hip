@@ -71,6 +71,10 @@ nmx_ctx *nmx_create(int device) {
         free(ctx);
         return nullptr;
     }
+    if (hipMalloc(&ctx->mix_ws, NMX_MIX_WS) != hipSuccess) {
+        ctx->mix_ws = nullptr;
+        (void)hipGetLastError(); /* not an error of the next launch */
+    }
     return ctx;
 }
 
@@ -78,6 +82,7 @@ void nmx_destroy(nmx_ctx *ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
+    (void)hipFree(ctx->mix_ws);
     (void)hipStreamDestroy(ctx->stream);
     free(ctx);
 }

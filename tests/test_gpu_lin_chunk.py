@@ -2,10 +2,10 @@
 the tokens in parallel, then kv chains and skewed o chains in waves of their own).
 
 The recurrence is compared with the oracle and the whole mixer with lin_mix_k, the one-launch kernel
-that takes the same pass when the intermediate buffers are left out. Bar: bit-exact for outputs,
-recurrent state and conv state. Sizes at the pipeline's edges: 9 tokens (less than the 15 steps a
-sum takes), 16 and 17 (one batch, one more token), 48, 63, 64 (the ring of 4 batches wraps), pending
-replays, shared key heads, dk 64 to 256, a last column group that is not 16 wide."""
+that takes the same pass under capture. Bar: bit-exact for outputs, recurrent state and conv state.
+Sizes at the pipeline's edges: 9 tokens (less than the 15 steps a sum takes), 16 and 17 (two batches
+of 8, one more token), 48, 63, 64 (the 8 batches that the ring holds), 209 and 512 (the ring wraps),
+pending replays, shared key heads, dk 64 to 256, a last column group that is not 16 wide."""
 from __future__ import annotations
 
 import ctypes
@@ -50,8 +50,14 @@ def test_rule_equals_oracle(dev, case):
     assert_bits_equal(state_from_dev(dS.numpy(), heads, dk, dv), want_S, "state")
 
 
+def chunk_fn(dev):
+    fn = dev.lib.nmx_lin_mix_chunk
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(LinMixArgs)]
+    return fn
+
+
 def one_launch(dev, c):
-    """The pass through lin_mix_k: no intermediate buffers."""
+    """The pass through lin_mix_k: a captured launch, which does not use the context's workspace."""
     n, heads, dk, dv, C = (c[k] for k in ("n", "heads", "dk", "dv", "C"))
     d = {k: dev.to_device(v) for k, v in c["host"].items()}
     nb = heads * dv // 32
@@ -63,9 +69,13 @@ def one_launch(dev, c):
                      p(d["A_log"]), None, p(d["dt_bias"]), None, None)
     rule = LinArgs(n, heads, 1, dk, dv, C, heads * dv, None, None, None, p(d["S"]), None, None,
                    p(d["pend"]), c["keep"], 0, None)
+    dev.graph_begin()
     dev.lin_mix(LinMixArgs(pre, rule, p(d["z"]), heads * dv, p(d["norm_w"]), 1e-6, p(y), heads * dv,
                            A8(p(aq), p(ad), p(afs))))
+    g = dev.graph_end()
+    dev.graph_launch(g)
     dev.sync()
+    dev.graph_destroy(g)
     return dict(aq=aq.numpy(), ad=ad.numpy(), afs=afs.numpy(), y=y.numpy(), S=d["S"].numpy(),
                 state=d["state"].numpy())
 
@@ -95,8 +105,7 @@ def test_long_chunk_equals_pieces(dev, case):
     64 over the same rows, the states carried from one to the next."""
     n, heads, rep, dk, dv, keep = case
     print(f"[case] lin long chunk {case}", flush=True)
-    fn = dev.lib.nmx_lin_mix_chunk
-    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(LinMixArgs)]
+    fn = chunk_fn(dev)
     c = make_case(dev, np.random.default_rng(n + dk), n, heads, rep, dk, dv, logged=False, keep=keep)
     h, C, vd = c["host"], c["C"], heads * dv
 
@@ -122,3 +131,82 @@ def test_long_chunk_equals_pieces(dev, case):
 
     for got, want, what in zip(passes(512), passes(64), ("y", "state", "conv state")):
         assert_bits_equal(got, want, what)
+
+
+def buffers(dev, c, fill):
+    """The mixer's arguments of nmx_lin_mix_chunk, every intermediate buffer filled with `fill`."""
+    n, heads, rep, dk, dv, C = c["n"], c["heads"], c["rep"], c["dk"], c["dv"], c["C"]
+    d, vd = {k: dev.to_device(v) for k, v in c["host"].items()}, heads * dv
+    mid = {k: dev.to_device(np.full((n, w), fill, np.float32))
+           for k, w in (("out", C), ("beta", heads), ("decay", heads), ("o", vd))}
+    y = dev.zeros((n, vd), np.float32)
+    pre = LinPreArgs(n, C, c["K"], dk, c["kd"], p(d["raw"]), C, p(mid["out"]), p(d["state"]),
+                     p(d["conv_w"]), None, np.float32(1.0 / np.sqrt(dk)), 1e-6, p(d["b"]), p(d["a"]),
+                     heads, heads, p(d["A_log"]), None, p(d["dt_bias"]), p(mid["beta"]), p(mid["decay"]))
+    rule = LinArgs(n, heads, rep, dk, dv, C, vd, p(mid["out"]), p(mid["decay"]), p(mid["beta"]),
+                   p(d["S"]), p(mid["o"]), None, p(d["pend"]), c["keep"], 0, None)
+    args = LinMixArgs(pre, rule, p(d["z"]), vd, p(d["norm_w"]), 1e-6, p(y), vd, A8(None, None, None))
+    return args, d, mid, y
+
+
+@pytest.mark.parametrize("n,keep", [(9, 0), (64, 3)])
+def test_mixer_leaves_buffers_untouched(dev, n, keep):
+    """nmx_lin_mix in the fused kernel's shapes does not use the caller's intermediate buffers, and the
+    results of two passes in a row (the context's workspace holds the first one's) are lin_mix_k's."""
+    print(f"[case] lin chunk mixer buffers n={n} keep={keep}", flush=True)
+    c = make_case(dev, np.random.default_rng(n + keep), n, 4, 1, 128, 128, logged=False, keep=keep)
+    want = one_launch(dev, c)
+    for _ in range(2):
+        args, d, mid, y = buffers(dev, c, -7.0)
+        dev.lin_mix(args)
+        dev.sync()
+        for k, b in mid.items():
+            assert (b.numpy() == -7.0).all(), f"{k} written"
+        for got, k in ((y, "y"), (d["S"], "S"), (d["state"], "state")):
+            assert_bits_equal(got.numpy(), want[k], k)
+
+
+@pytest.mark.parametrize("n", [9, 64])
+def test_overlapping_buffers_take_one_launch(dev, n):
+    """nmx_lin_mix_chunk of at most 64 rows whose o lies in the raw inputs: lin_mix_k, or the chunk
+    kernels over the context's workspace; the same bits, and the raw inputs untouched."""
+    print(f"[case] lin chunk mixer overlap n={n}", flush=True)
+    c = make_case(dev, np.random.default_rng(n), n, 4, 1, 128, 128, logged=False)
+    want = one_launch(dev, c)
+    args, d, mid, y = buffers(dev, c, 0.0)
+    args.rule.o = p(d["raw"])
+    dev.check(chunk_fn(dev)(dev.ctx, ctypes.byref(args)))
+    dev.sync()
+    assert_bits_equal(d["raw"].numpy(), c["host"]["raw"], "raw inputs")
+    for got, k in ((y, "y"), (d["S"], "S"), (d["state"], "state")):
+        assert_bits_equal(got.numpy(), want[k], k)
+
+
+def test_long_chunk_refusals(dev):
+    """Above 64 rows nmx_lin_mix_chunk refuses on the host what only the other kernels take; n is
+    also bounded by NMX_CHUNK_ROWS, and by 64 in nmx_lin_mix."""
+    print("[case] lin chunk refusals", flush=True)
+    c = make_case(dev, np.random.default_rng(1), 65, 2, 1, 128, 128, logged=False)
+    log = dev.zeros((65, 2, 257), np.float32)
+
+    def change(args, d, mid, what):
+        if what == "log":
+            args.rule.log = p(log)
+        elif what == "no o":
+            args.rule.o = None
+        elif what == "o in raw":
+            args.rule.o = p(d["raw"])
+        elif what == "qkv elsewhere":
+            args.rule.qkv = p(d["raw"])
+        elif what == "513 rows":
+            args.pre.n = args.rule.n = 513
+
+    for what in ("log", "no o", "o in raw", "qkv elsewhere", "513 rows"):
+        args, d, mid, y = buffers(dev, c, 0.0)
+        change(args, d, mid, what)
+        assert chunk_fn(dev)(dev.ctx, ctypes.byref(args)) == -1, what
+        assert b"nmx_lin_mix" in dev.lib.nmx_error(dev.ctx)
+        dev.sync()
+        assert_bits_equal(d["S"].numpy(), c["host"]["S"], "state")
+    args, d, mid, y = buffers(dev, c, 0.0)
+    assert dev.lib.nmx_lin_mix(dev.ctx, ctypes.byref(args)) == -1
