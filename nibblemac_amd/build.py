@@ -36,13 +36,14 @@ ARCH = "gfx950"
 # hipcc default, kept), and no packed-fp32 code generation. Kernel arguments preloaded into
 # SGPRs (the leading pointer / integer arguments, up to 16 SGPRs; the code object keeps the
 # loading prologue for firmware without preloading), so a kernel's first memory requests do
-# not wait for a load from the argument segment.
+# not wait for a load from the argument segment. A kernel that misses the occupancy it asks for
+# (amdgpu_waves_per_eu) does not build: its workgroups would wait for each other on the device.
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-fno-gpu-flush-denormals-to-zero", "-fno-fast-math",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
-    "-Wall", "-Wno-unused-function", f"-I{INCLUDE}", f"-I{HIP_DIR}",
+    "-Wall", "-Wno-unused-function", "-Werror=pass-failed", f"-I{INCLUDE}", f"-I{HIP_DIR}",
 ]
 C_FLAGS = ["-O2", "-std=c11", "-ffp-contract=off", "-fPIC", "-Wall", "-Wextra",
            "-Wno-unused-parameter", f"-I{INCLUDE}", f"-I{HOST_DIR}", "-pthread"]

@@ -309,25 +309,31 @@ __global__ __launch_bounds__(512) void attn_pvc_k(const float *__restrict__ wts,
 /* Softmax and P.V of a few rows in caches past 8192 positions (steps and verify passes): workgroup =
  * (32 dims, head, token). Each forms its row's max and sum itself (attn_sm_k's steps; the 8 workgroups
  * of a row run them side by side, and a separate launch would cost a short context 2 us), then wave
- * 0's lanes run the P.V chains, one per dim. The chain, one dependent add per position, bounds it (8.1
- * clocks a step: 68 us for 20000 positions), so everything else runs beside it: waves 1-4 store tile
- * i + 1's products w_p v_p[d] in LDS, one row per dim, while wave 0 adds tile i, and have tile i + 2's
- * values and scores in flight. One token at 20000 positions, binary16 cache: 130 us (one kernel that
- * stored each tile between two runs of the chains: 429 us). Up to PL_SHORT positions a row is one pass:
- * layers of 1 token at 50, 3 at 120, 5 at 900 positions take 34.3, 38.6, 57.9 us (34.8, 39.9, 58.1),
- * 5 at 1500 63.4 (70.4); 8 tokens, 512 workgroups of five waves, lose 1.5 us there (8 at 300: 55.8,
- * 54.4) and gain past it. */
+ * 0's lanes run the P.V chains, one per dim. The chain, one dependent add per position, bounds it (68
+ * us for 20000 positions), so everything else runs beside it: waves 1-4 store tile i + 1's products
+ * w_p v_p[d] in LDS, one row per dim, while wave 0 adds tile i, and have tile i + 2's values and scores
+ * in flight. One token at 20000 positions, binary16 cache: 130 us (one kernel that stored each tile
+ * between two runs of the chains: 429 us). Up to PL_SHORT positions a row is one pass.
+ * 5 rows of 8 heads are 320 workgroups and 8 rows 512, two to a CU, whose 10 waves fit its SIMDs only
+ * at 128 registers; at 140 (tiles of 440 positions in the short pass) the second one waited for the
+ * first: 6.6 against 4.4 us for 5 rows at 40 positions, 23.6 against 14.8 us for 8 at 1000. Whole
+ * layers of 1 token at 50, 5 at 40, 5 at 900, 8 at 300 and 8 at 3000 positions: 34.2, 41.5, 49.9, 51.9
+ * and 78.5 us (34.8, 42.2, 58.2, 54.5 and 109.6 with the kernel that alternated). */
 constexpr int PL_P = 256;        /* positions per tile */
 constexpr int PL_D = 32;         /* output dims per workgroup: one A8 block */
 constexpr int PL_RS = PL_P + 4;  /* row stride: 16-byte aligned, 4 words apart modulo 64 banks */
 constexpr int PL_SHORT = 1024;   /* positions up to which a row is one pass without the pipeline */
-constexpr int PS_P = 440;        /* positions per tile there: 11 values per thread, none left over */
+constexpr int PS_P = 240;        /* positions per tile there: 6 values per thread, none left over */
+constexpr int PL_LDS = 2 * PL_D * PL_RS * 4;
 
 template <int KVT>
-__global__ __launch_bounds__(320) void attn_pvl_k(const float *__restrict__ sc, Attn a) {
+__global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(4))) void attn_pvl_k(
+    const float *__restrict__ sc, Attn a) {
     constexpr int F4 = PL_D / 4, PER = PL_P * F4 / 256, T = 320;
-    /* the softmax's two segments, then the two tiles of products */
-    __shared__ __align__(16) float buf[2 * PL_D * PL_RS];
+    /* the softmax's two segments, then the two tiles of products: PL_LDS bytes, dynamic, as the
+     * compiler would count two workgroups per CU and not keep to the registers of four waves */
+    extern __shared__ float4 smem4[];
+    float *buf = (float *)smem4;
     static_assert(4 * SM_S4 <= PL_D * PL_RS, "a segment fits in a tile's place");
     __shared__ float red[8];
     const int hd = a.hd, rep = a.nh / a.nkv, S = (hd / PL_D) * a.nkv, tid = threadIdx.x;
@@ -525,15 +531,25 @@ int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
     return 0;
 }
 
+template <int KVT>
+int launch_long(nmx_ctx *ctx, const Attn &a, const float *sc) {
+    static bool ready = false; /* idempotent */
+    if (!ready) {
+        NMX_HIP(ctx, hipFuncSetAttribute((const void *)attn_pvl_k<KVT>,
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, PL_LDS));
+        ready = true;
+    }
+    attn_pvl_k<KVT><<<(unsigned)((a.hd / PL_D) * a.nh * a.n), 320, PL_LDS, ctx->stream>>>(sc, a);
+    NMX_LAUNCHED(ctx, "attn_pvl");
+    return 0;
+}
+
 } // namespace
 
 int nmx_attn_long(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, const float *sc) {
-    const unsigned pg = (unsigned)((a.hd / PL_D) * a.nh * a.n);
-    if (kv_dtype == KV_F16) attn_pvl_k<KV_F16><<<pg, 320, 0, ctx->stream>>>(sc, a);
-    else if (kv_dtype == KV_I8) attn_pvl_k<KV_I8><<<pg, 320, 0, ctx->stream>>>(sc, a);
-    else attn_pvl_k<KV_F32><<<pg, 320, 0, ctx->stream>>>(sc, a);
-    NMX_LAUNCHED(ctx, "attn_pvl");
-    return 0;
+    if (kv_dtype == KV_F16) return launch_long<KV_F16>(ctx, a, sc);
+    if (kv_dtype == KV_I8) return launch_long<KV_I8>(ctx, a, sc);
+    return launch_long<KV_F32>(ctx, a, sc);
 }
 
 int nmx_attn_chunk(nmx_ctx *ctx, const nmx_attn_dev &a, int kv_dtype, float *sc) {
