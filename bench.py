@@ -22,7 +22,8 @@ MALL (one copy). `kernels` holds configs 1-4 (nibblemac_amd/kbench.py). `cpu_bas
 reference engine's own sources with the oracle's threaded Q4K operators
 (oracle/_ref/libpinfer_refq4k.so) on the host cores: the config-5 workload itself on the GPU
 box's CPU share (16 threads), its tokens checked against the GPU's, plus a 1-thread run on a
-bounded sample and the oracle's Q4K matvec of config 1 on 1 thread. With random weights the
+bounded sample and the oracle's Q4K matvec of config 1 on 1 thread; null where that library is
+not built. With random weights the
 drafts are essentially never accepted; `accepting` times the same workload on the same weights
 with final norms that make the drafts agree (multi-token commits and deferred DeltaNet replays),
 its tokens checked against plain greedy decoding.
@@ -179,12 +180,16 @@ def head_eager(dev: Device, copies: int, reps: int = 40) -> dict:
     return {"us_per_call": round(dev.elapsed_ms(e0, e1) / reps * 1e3, 2), "timing": "eager"}
 
 
-def cpu_baseline(path: Path, gpu_run: tuple, prompt: np.ndarray) -> dict:
+def cpu_baseline(path: Path, gpu_run: tuple, prompt: np.ndarray) -> dict | None:
     """The reference engine on the host: the config-5 workload on CPU_SHARE threads (tokens and
     statistics checked against the GPU's), a 1-thread run of a bounded sample, and the
-    oracle's config-1 matvec on 1 thread."""
+    oracle's config-1 matvec on 1 thread. None where the reference engine is not built (its
+    sources are not here)."""
     from oracle import refengine  # the checker and CPU baseline live with the oracle
 
+    if not refengine.REFQ4K.exists():
+        log(f"cpu baseline skipped: {refengine.REFQ4K} is not built")
+        return None
     thr, aff = host_threads()
     full = refengine.bench_generate(path, prompt, N_GEN, K_DRAFT, DRAFT_VOCAB, thr)
     gtoks, gst = gpu_run
