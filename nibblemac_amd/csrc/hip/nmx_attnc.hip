@@ -322,7 +322,10 @@ __global__ __launch_bounds__(512) void attn_pvc_k(const float *__restrict__ wts,
 constexpr int PL_P = 256;        /* positions per tile */
 constexpr int PL_D = 32;         /* output dims per workgroup: one A8 block */
 constexpr int PL_RS = PL_P + 4;  /* row stride: 16-byte aligned, 4 words apart modulo 64 banks */
-constexpr int PL_SHORT = 1024;   /* positions up to which a row is one pass without the pipeline */
+/* Positions up to which a row is one pass without the pipeline. us of the kernel at 1, 5 and 8 rows,
+ * one pass against pipeline: 300 positions 6.8, 6.9, 7.2 against 7.6, 8.9, 9.3; 600: 9.8, 10.6, 10.7
+ * against 9.8, 11.6, 12.0; 1000: 13.4, 14.6, 14.7 against 12.1, 14.1, 14.5. */
+constexpr int PL_SHORT = 768;
 constexpr int PS_P = 240;        /* positions per tile there: 6 values per thread, none left over */
 constexpr int PL_LDS = 2 * PL_D * PL_RS * 4;
 

@@ -100,7 +100,8 @@ def widen(cache, kvt, nkv, ctx, wide, hd):
     # n, query heads, KV heads, head size, kv dtype, position of token 0
     (1, 8, 2, 256, 1, 8000), (5, 8, 2, 256, 0, 4094), (8, 4, 4, 64, 2, 250), (3, 6, 2, 128, 0, 0),
     (1, 8, 2, 256, 2, 255), (2, 8, 2, 256, 0, 511), (3, 8, 2, 256, 1, 438), (8, 8, 2, 256, 0, 1020),
-    (3, 8, 2, 256, 2, 238), (5, 8, 2, 256, 1, 477), (8, 8, 2, 256, 0, 956),  # the 240-position tiles
+    (3, 8, 2, 256, 2, 238), (5, 8, 2, 256, 1, 477), (8, 8, 2, 256, 0, 716),  # the 240-position tiles
+    (8, 8, 2, 256, 0, 763), (3, 8, 2, 256, 2, 1022),  # rows of one pass and of the pipeline
 ], ids=lambda c: "n%d_h%d_%d_hd%d_kv%d_pos%d" % c)
 def test_long_cache_equals_in_lds(dev, case):
     """A cache past 8192 positions (softmax in segments, P.V products made beside the
