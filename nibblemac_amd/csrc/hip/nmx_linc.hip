@@ -4,8 +4,10 @@
  * operation for operation; the gated norm after it is nmx_lin_post's kernel.
  *
  * The recurrence is one chain per value column: per token kv = sum of 128 keys in order, then
- * delta, then the state, which the next token's kv needs. A dependent add takes 8.1 clocks, so a
- * token takes at least 128 of them (0.43 us) whatever the layout. Three things are moved out of
+ * delta, then the state, which the next token's kv needs. A dependent add on registers takes 4.25
+ * clocks (1.78 ns), 5.16 on average with a hand-over to the next lane every 8, so the adds of a token
+ * are 0.28 us; it takes 0.40 (the slope from 256 to 512 tokens), the rest being the products, the
+ * broadcast of kv, delta, the state's update and the operands' reads. Three things are moved out of
  * that chain's way:
  *   - o_t = sum of S_t q_t is a chain of its own, but nothing waits for it: other waves run it,
  *     on a copy of the state that they advance from the published deltas. There the 16 lanes of a
@@ -16,8 +18,8 @@
  *   - 8 columns per workgroup of 4 waves (two on the kv chains, two on o): one wave per SIMD, 256
  *     workgroups at 16 heads x 128 columns, where lin_mix_k's one workgroup per head left 240 CUs
  *     idle and put two chain waves on each SIMD.
- * 64 tokens, 16 heads x 128 x 128: 36.3 us, 500 tokens 210 us, 0.41 us per token (lin_mix_k, conv and
- * gated norm included: 97-100 us for 64, 1.45 us per token). */
+ * 64 tokens, 16 heads x 128 x 128: 34.3 us, 512 tokens 215 us (lin_mix_k, conv and gated norm
+ * included: 97-100 us for 64, 1.45 us per token). */
 #include "nmx_internal.h"
 #include "nmx_linc.h"
 #include "nmx_lanes.h"
@@ -103,9 +105,10 @@ __global__ __launch_bounds__(256) void lin_prec_k(nmx_lin_pre_args a) {
 
 /* Tokens run in batches of TB (one barrier, one staged batch each). The o chains end a batch and 15
  * steps after the kv chains, which restart their operand reads at every batch: batches of 8 for
- * chunks of up to RC_SHORT tokens, where the end counts (45 tokens 27.5 us, 31.3 in batches of 16; 64
- * tokens 36.3 and 39.8), of 16 above (500 tokens 210 us, 212 in batches of 8). */
-constexpr int RC_SHORT = 192;
+ * chunks of up to RC_SHORT tokens, where the end counts, of 16 above. us in batches of 8 and of 16:
+ * 64 tokens 34.3 and 37.4, 192 86.2 and 87.6, 256 111.9 and 113.0, 320 138.1 and 137.9, 512 216.0 and
+ * 214.7. */
+constexpr int RC_SHORT = 256;
 constexpr int RC_JW = 8;   /* value columns per workgroup */
 constexpr int RC_TOK = 64; /* tokens in LDS: a batch being staged, one in the kv chains, those of the
                             * last 15 steps in the o chains */

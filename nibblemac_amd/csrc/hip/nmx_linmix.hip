@@ -445,7 +445,7 @@ int launch_mix(nmx_ctx *ctx, const LinMix &m, size_t lds) {
 /* Whether the chunk kernels (nmx_linc.hip) take the mixer with these intermediate buffers: more
  * than 8 tokens without a log, and buffers that overlap nothing that a later kernel reads or writes.
  * They are the caller's where the caller gave them to be written (nmx_lin_mix_chunk, and the shapes
- * outside the fused kernel), else the context's. 64 tokens, 16 heads of 128: 4.6 + 36.3 + 4.7 us
+ * outside the fused kernel), else the context's. 64 tokens, 16 heads of 128: 4.6 + 34.3 + 4.7 us
  * against 97-100 us for lin_mix_k, whose time per token is 1.45 us above about 5 us of setup. */
 bool chunk_ok(const nmx_lin_mix_args &a) {
     const nmx_lin_pre_args &p = a.pre;

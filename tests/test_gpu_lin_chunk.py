@@ -98,10 +98,11 @@ def test_mixer_equals_one_launch(dev, case):
 
 @pytest.mark.parametrize("case", [
     # n, heads, rep, dk, dv, keep
-    (193, 2, 1, 256, 64, 3), (192, 4, 2, 128, 32, 0), (209, 2, 1, 64, 64, 0), (512, 2, 2, 128, 32, 0),
+    (257, 2, 1, 256, 64, 3), (256, 4, 2, 128, 32, 0), (273, 2, 1, 64, 64, 0), (512, 2, 2, 128, 32, 0),
+    (209, 2, 1, 128, 32, 2),
 ], ids=lambda c: "n%d_h%d_rep%d_dk%d_dv%d_keep%d" % c)
 def test_long_chunk_equals_pieces(dev, case):
-    """nmx_lin_mix_chunk above 64 rows (batches of 8 up to 192 tokens, of 16 above) against passes of
+    """nmx_lin_mix_chunk above 64 rows (batches of 8 up to 256 tokens, of 16 above) against passes of
     64 over the same rows, the states carried from one to the next."""
     n, heads, rep, dk, dv, keep = case
     print(f"[case] lin long chunk {case}", flush=True)
