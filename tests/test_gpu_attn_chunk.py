@@ -7,6 +7,8 @@ at the tiles' edges: 9 rows, ragged row groups (3 heads per KV group), 64-positi
 left inside the chunk, softmax segments of 4096, caches past 8192 positions, head sizes 64 to 512."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -17,9 +19,15 @@ from tests.test_gpu_q4k import assert_bits_equal
 pytestmark = pytest.mark.gpu
 
 
-def passes(dev, host, shape, step):
+def fused_chunk(dev):
+    fn = dev.lib.nmx_attn_fused_chunk
+    fn.restype, fn.argtypes = ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(AttnArgs), ctypes.c_int]
+    return fn
+
+
+def passes(dev, host, shape, step, score_rows=0):
     """The chunk in passes of `step` tokens: o [n][nh hd], its A8 (codes, d, fsum per block and
-    token), the caches."""
+    token), the caches. score_rows: through nmx_attn_fused_chunk with a workspace of so many rows."""
     n, nh, nkv, hd, max_ctx, kvt, pos0 = shape
     kc, vc = dev.to_device(host["kc"]), dev.to_device(host["vc"])
     const = {k: dev.to_device(host[k]) for k in ("q_norm", "k_norm", "cos", "sin")}
@@ -31,13 +39,16 @@ def passes(dev, host, shape, step):
         o = dev.zeros((m, nh * hd), np.float32)
         a8 = (dev.zeros((nb, m, 32), np.int8), dev.zeros((nb, m), np.float32),
               dev.zeros((nb, m), np.float32))
-        sc = dev.zeros((m, nh, max_ctx), np.float32)
+        sc = dev.zeros((score_rows or m, nh, max_ctx), np.float32)
         a = AttnArgs(m, nh, nkv, hd, hd // 4, max_ctx, q.ptr, k.ptr, v.ptr, const["q_norm"].ptr,
                      const["k_norm"].ptr, 1e-6, np.float32(1.0 / np.sqrt(hd)), const["cos"].ptr,
                      const["sin"].ptr, kc.ptr, vc.ptr, pos.ptr, t0 - 3, o.ptr,
                      A8(*[b.ptr for b in a8]), sc.ptr, kvt)
-        dev.attn_prep(a)
-        dev.attn(a)
+        if score_rows:
+            dev.check(fused_chunk(dev)(dev.ctx, ctypes.byref(a), score_rows))
+        else:
+            dev.attn_prep(a)
+            dev.attn(a)
         dev.sync()
         outs.append((o.numpy(), *[b.numpy() for b in a8]))
         for b in (q, k, v, pos, o, *a8, sc):
@@ -63,13 +74,10 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: "n%d_h%d_%d_hd%d_ctx%d_kv%d_pos%d" % c)
-def test_chunk_equals_steps(dev, case):
-    n, nh, nkv, hd, max_ctx, kvt, pos0 = case
-    print(f"[case] attn chunk {case}", flush=True)
-    rng = np.random.default_rng(n + 7 * hd + pos0)
+def make_host(rng, case):
+    n, nh, nkv, hd, max_ctx, kvt, _ = case
     ang = rng.uniform(0, 2 * np.pi, (max_ctx, hd // 8))
-    host = dict(
+    return dict(
         q=rng.standard_normal((n, nh, 2 * hd)).astype(np.float32),
         k_in=rng.standard_normal((n, nkv * hd)).astype(np.float32),
         v_in=rng.standard_normal((n, nkv * hd)).astype(np.float32),
@@ -78,10 +86,48 @@ def test_chunk_equals_steps(dev, case):
         cos=np.cos(ang).astype(np.float32), sin=np.sin(ang).astype(np.float32),
         kc=cache_bytes(rng, kvt, nkv, max_ctx, hd), vc=cache_bytes(rng, kvt, nkv, max_ctx, hd),
     )
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "n%d_h%d_%d_hd%d_ctx%d_kv%d_pos%d" % c)
+def test_chunk_equals_steps(dev, case):
+    n, nh, nkv, hd, max_ctx, kvt, pos0 = case
+    print(f"[case] attn chunk {case}", flush=True)
+    host = make_host(np.random.default_rng(n + 7 * hd + pos0), case)
     want = passes(dev, host, case, 8)
     got = passes(dev, host, case, 64)
     for k in want:
         assert_bits_equal(got[k], want[k], k)
+
+
+@pytest.mark.parametrize("case,score_rows", [
+    ((130, 8, 2, 256, 512, 0, 20), 64),   # two whole slices and one of two rows
+    ((512, 4, 2, 64, 640, 1, 100), 200),  # the most rows, a ragged last slice
+    ((9, 6, 2, 128, 256, 2, 50), 4),      # fewer workspace rows than a pass of steps
+], ids=lambda c: str(c).replace(" ", ""))
+def test_slices_equal_steps(dev, case, score_rows):
+    """nmx_attn_fused_chunk in slices of the scores workspace's rows."""
+    print(f"[case] attn chunk slices {case} {score_rows}", flush=True)
+    host = make_host(np.random.default_rng(sum(case)), case)
+    want = passes(dev, host, case, 8)
+    got = passes(dev, host, case, 512, score_rows)
+    for k in want:
+        assert_bits_equal(got[k], want[k], k)
+
+
+def test_fused_chunk_refusals(dev):
+    """On the host: a workspace of no rows or none at all, and more rows than NMX_CHUNK_ROWS."""
+    print("[case] attn chunk refusals", flush=True)
+    b = dev.zeros(1 << 18, np.float32)
+    pos = dev.zeros(1, np.int32)
+
+    def args(n, scores):
+        return AttnArgs(n, 2, 1, 64, 16, 64, b.ptr, b.ptr, b.ptr, b.ptr, b.ptr, 1e-6, np.float32(0.125),
+                        b.ptr, b.ptr, b.ptr, b.ptr, pos.ptr, 0, b.ptr, A8(None, None, None), scores, 0)
+
+    for n, scores, rows in ((16, b.ptr, 0), (16, None, 4), (16, None, 16), (4, None, 4), (513, b.ptr, 64)):
+        assert fused_chunk(dev)(dev.ctx, ctypes.byref(args(n, scores)), rows) == -1, (n, scores, rows)
+    dev.sync()
+    assert not b.numpy().any()
 
 
 def widen(cache, kvt, nkv, ctx, wide, hd):

@@ -12,6 +12,7 @@ import pytest
 
 import oracle
 from nibblemac_amd import pqtool
+from nibblemac_amd.nmx import A8, NormIn
 from tests.test_gpu_q4k import assert_bits_equal
 
 pytestmark = pytest.mark.gpu
@@ -36,12 +37,14 @@ def chunk(dev, Ws, rows, cols, n, q, d, fs, pad):
 
 CASES = [
     # rows of each matrix, cols, vectors, output row padding
-    ((16,), 256, 9, 0), ((8192,), 256, 17, 0),            # 512 and 1024 workgroups' worth
-    ((8208,), 256, 16, 1), ((12,), 512, 33, 0),
+    ((16,), 256, 9, 0), ((8192,), 256, 16, 0),             # one tile; 512, the last of q4k_mm_k
+    ((8208,), 256, 16, 1), ((8192,), 256, 17, 0),          # 513 and 1024 of q4k_mmn_k
+    ((12,), 512, 33, 0),
     ((4096, 20, 4), 768, 48, 0), ((1024,), 1280, 500, 0),  # three waves; five
     ((1024,), 2048, 257, 0), ((520,), 2304, 320, 3),       # 8 waves; 9 superblocks in two rounds
     ((2052,), 3584, 70, 0), ((600,), 4352, 300, 0),        # two rounds of 7; three of 6, 6, 5
     ((7168,), 1024, 512, 0), ((64,), 1024, 512, 0),
+    ((2080,), 4096, 512, 0),  # 32 tiles per workgroup in two rounds: the most LDS
 ]
 
 
@@ -64,3 +67,26 @@ def test_tiles_equal_oracle(dev, case):
         assert not y[:, r:].any(), "padding columns written"
     for b in (*dWs, dq, dd, df):
         b.free()
+
+
+def test_more_than_512_rows_refused(dev):
+    """On the host, before anything is enqueued: the three matmul calls for chunks of rows."""
+    print("[case] mm chunk refusals", flush=True)
+    vp, i = ctypes.c_void_p, ctypes.c_int
+    n, cols, rows = 513, 256, 32
+    W, X = dev.zeros(rows // 4 * 576, np.uint8), dev.zeros((n, cols), np.float32)
+    q, d, fs = dev.zeros((8, n, 32), np.int8), dev.zeros((8, n), np.float32), dev.zeros((8, n), np.float32)
+    a8 = A8(q.ptr, d.ptr, fs.ptr)
+    Y = [dev.zeros((n, rows), np.float32) for _ in range(2)]
+    norm = NormIn(X.ptr, cols, None, 0, None, 0, X.ptr, 1e-6)
+    one = ((vp * 1)(W.ptr), (i * 1)(rows), (vp * 1)(Y[0].ptr), (i * 1)(rows))
+    mm, mmn, glu = (getattr(dev.lib, f"nmx_q4k_{x}_chunk") for x in ("matmul", "matmul_norm", "swiglu"))
+    mmn.argtypes = [vp, i, vp, vp, vp, vp, i, i, ctypes.POINTER(NormIn), A8]
+    glu.argtypes = [vp, vp, vp, i, i, i, vp, vp, vp, ctypes.POINTER(NormIn), vp, A8, A8, vp, vp]
+    mm.argtypes = [vp, i, vp, vp, vp, vp, i, i, vp, vp, vp]
+    assert mm(dev.ctx, 1, *one, cols, n, q.ptr, d.ptr, fs.ptr) == -1
+    assert mmn(dev.ctx, 1, *one, cols, n, ctypes.byref(norm), a8) == -1
+    assert glu(dev.ctx, W.ptr, W.ptr, rows, cols, n, q.ptr, d.ptr, fs.ptr, None, None, a8, a8, Y[0].ptr,
+               Y[1].ptr) == -1
+    dev.sync()
+    assert not Y[0].numpy().any()
