@@ -79,7 +79,8 @@ int nmx_quant_a8(nmx_ctx *ctx, const float *X, int n, int cols, int8_t *q, float
  * W: .pq Q4K_G32 bytes [rows/4][cols/256][576] on the device (rows % 4 == 0, cols % 256 == 0).
  * A8 inputs as nmx_quant_a8 writes them for n vectors. Y [n][y_stride] fp32 (y_stride >= rows).
  * dots (may be NULL): int32 sub-block sums [n][rows][cols/32] (exactness checks).
- * n: 1..64 (split into register passes of <= 8 vectors; results do not depend on n).
+ * n: 1..64 (one register pass of <= 8 vectors, more on the matrix cores in tiles of 16; results do
+ * not depend on n).
  */
 int nmx_q4k_matmul(nmx_ctx *ctx, const void *W, int rows, int cols, int n, const int8_t *q,
                    const float *d, const float *fsum, float *Y, int y_stride, int32_t *dots);

@@ -55,12 +55,14 @@ constexpr int PV_W = 8;      /* rows per P.V workgroup: one per wave */
 constexpr int SM_SEG = 4096; /* positions per softmax segment in LDS */
 constexpr int SM_S4 = SM_SEG / 4 + 4; /* row stride of a segment's four partial sums */
 
-/* Scores. Lane = position; a wave takes 4 rows at a time, whose query elements are scalars, and
- * keeps the 16 interleaved partial sums of each in registers: per 16 elements 4 LDS reads of the
- * position's key (shared by the 4 rows) feed 128 VALU instructions. Tile rows are hd + 4 floats
- * apart, so 16 lanes' 16-byte reads cover the banks once. 64 tokens at 4000 positions, int8
- * cache: 45.2 us; over a 2000-token fp32 prompt 22.9 us on average. attn_score_k, one token x 32
- * positions per workgroup and so a key tile per token: 96.7 and 34.8 us. */
+/* Scores. Lane = position; a wave takes 4 rows at a time, whose query elements it holds 16 to a row
+ * of lanes and broadcasts in the multiply, and keeps the 16 interleaved partial sums of each in
+ * registers: per 16 elements 4 LDS reads of the position's key (shared by the 4 rows) feed 128 VALU
+ * instructions. Tile rows are hd + 4 floats apart, so 16 lanes' 16-byte reads cover the banks once.
+ * 64 tokens at 4000 positions, int8 cache: 45.5 us (attn_score_k, one token x 32 positions per
+ * workgroup and so a key tile per token: 96.7); a 45-token prompt 18.6 us, a 2000-token fp32 prompt
+ * in slices of 256 tokens 67.5 us each on average. A query element is requested one step of 16 dims
+ * ahead only, which few waves per SIMD do not hide. */
 template <int KVT>
 __global__ __launch_bounds__(512) void attn_scc_k(Attn a, float *__restrict__ sc) {
     extern __shared__ float4 smem4[];
@@ -205,14 +207,14 @@ __global__ __launch_bounds__(SM_T) void attn_sm_k(Attn a, float *__restrict__ sc
 }
 
 /* P.V, the output gate and A8. Lane = output dim, wave = row: a lane's chain is o = o + w_p v_p[d]
- * over its row's positions, w_p a scalar, v_p[d] from the tile that the 8 rows of the workgroup
- * share. 64 tokens x 8 heads fill 256 workgroups of 8 waves, two waves per SIMD, which is what a
- * SIMD needs to issue every cycle; a wave of two rows would halve the LDS reads and the waves.
- * Consecutive workgroups take different (dims, group) slices, so a slice of V stays in one XCD's
- * L2. 64 tokens at 4000 positions, int8 cache: 69 us (99 with weights and values requested one
- * 64-position tile ahead); over a 2000-token fp32 prompt 18.9 us on average. With attn_sm_k that
- * replaces attn_pv_k (32 dims x 1 token per workgroup, every product through LDS to one chain
- * wave): 934 and 191 us. */
+ * over its row's positions, w_p held 16 to a row of lanes and broadcast in the multiply, v_p[d] from
+ * the tile that the 8 rows of the workgroup share. 64 tokens x 8 heads fill 256 workgroups of 8 waves,
+ * two waves per SIMD, which is what a SIMD needs to issue every cycle; a wave of two rows would halve
+ * the LDS reads and the waves (54 against 52 us). Consecutive workgroups take different (dims, group)
+ * slices, so a slice of V stays in one XCD's L2. 64 tokens at 4000 positions, int8 cache: 69.7 us (99
+ * with weights and values requested one 64-position tile ahead); a 2000-token fp32 prompt in slices
+ * of 256 tokens 52 us each on average. With attn_sm_k that replaces attn_pv_k (32 dims x 1 token per
+ * workgroup, every product through LDS to one chain wave): 934 us at the first size. */
 template <int KVT>
 __global__ __launch_bounds__(512) void attn_pvc_k(const float *__restrict__ wts, Attn a) {
     constexpr int F4 = PV_D / 4, PER = PV_P * F4 / 512;
@@ -309,8 +311,9 @@ __global__ __launch_bounds__(512) void attn_pvc_k(const float *__restrict__ wts,
 /* Softmax and P.V of a few rows in caches past 8192 positions (steps and verify passes): workgroup =
  * (32 dims, head, token). Each forms its row's max and sum itself (attn_sm_k's steps; the 8 workgroups
  * of a row run them side by side, and a separate launch would cost a short context 2 us), then wave
- * 0's lanes run the P.V chains, one per dim. The chain, one dependent add per position, bounds it (68
- * us for 20000 positions), so everything else runs beside it: waves 1-4 store tile i + 1's products
+ * 0's lanes run the P.V chains, one per dim. The chain, one dependent add per position fed from LDS,
+ * bounds it (8.2 clocks a step in tiles of 256, 68 us for 20000 positions; on registers 4.25), so
+ * everything else runs beside it: waves 1-4 store tile i + 1's products
  * w_p v_p[d] in LDS, one row per dim, while wave 0 adds tile i, and have tile i + 2's values and scores
  * in flight. One token at 20000 positions, binary16 cache: 130 us (one kernel that stored each tile
  * between two runs of the chains: 429 us). Up to PL_SHORT positions a row is one pass.

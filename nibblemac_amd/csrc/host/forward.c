@@ -93,7 +93,7 @@ static int attn_block(pinfer_ctx *c, const e_layer *L, int n, void *kc, void *vc
     nmx_attn_args a = {n, c->n_heads, c->n_kv, hd, c->rot, c->max_ctx, s->ta, s->tb, s->tc,
                        L->q_norm, L->k_norm, c->rms_eps, 1.0f / sqrtf((float)hd), c->rope_cos,
                        c->rope_sin, kc, vc, c->ctl, pos_off, s->to, s->a_w, s->sc, c->kv_dtype};
-    CK(nmx_attn_fused_chunk(D, &a, c->score_rows)); /* prep + scores in one launch, then P.V */
+    CK(nmx_attn_fused_chunk(D, &a, c->score_rows)); /* up to 8 rows: prep + scores in one launch */
     return proj(c, &L->o, H, c->n_heads * hd, n, s->a_w, s->out);
 }
 
@@ -140,7 +140,7 @@ static int lin_block(pinfer_ctx *c, const e_layer *L, int n, int logged, const n
                       s->beta, c->rec + (size_t)li * nv * c->lk_dim * c->lv_dim, s->to,
                       logged ? c->log + (size_t)li * lrow : NULL, c->pend + (size_t)li * lrow,
                       c->cap - 1, 0, c->ctl + 2};
-    /* conv + gates, recurrence, gated norm + A8 of o: one launch */
+    /* conv + gates, recurrence, gated norm + A8 of o: one launch, or three for a prompt's rows */
     nmx_lin_mix_args m = {p, a, s->tb, vd, L->lin_norm, c->rms_eps, NULL, 0, s->a_w};
     CK(nmx_lin_mix_chunk(D, &m));
     return proj(c, &L->out, H, vd, n, s->a_w, s->out);
