@@ -518,13 +518,8 @@ template <int KVT>
 int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
     const int rows = a.n * (a.nh / a.nkv);
     const size_t lds = (size_t)SC_P * (a.hd + 4) * 4;
-    static bool ready = false; /* idempotent */
-    if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)attn_scc_k<KVT>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         SC_P * (512 + 4) * 4));
-        ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)attn_scc_k<KVT>, SC_P * (512 + 4) * 4, lds_set)) return -1;
     const dim3 sgrid((unsigned)((a.max_ctx + SC_P - 1) / SC_P),
                      (unsigned)((rows + SC_ROWS - 1) / SC_ROWS), (unsigned)a.nkv);
     attn_scc_k<KVT><<<sgrid, 512, lds, ctx->stream>>>(a, sc);
@@ -539,12 +534,8 @@ int launch_chunk(nmx_ctx *ctx, const Attn &a, float *sc) {
 
 template <int KVT>
 int launch_long(nmx_ctx *ctx, const Attn &a, const float *sc) {
-    static bool ready = false; /* idempotent */
-    if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)attn_pvl_k<KVT>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, PL_LDS));
-        ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)attn_pvl_k<KVT>, PL_LDS, lds_set)) return -1;
     attn_pvl_k<KVT><<<(unsigned)((a.hd / PL_D) * a.nh * a.n), 320, PL_LDS, ctx->stream>>>(sc, a);
     NMX_LAUNCHED(ctx, "attn_pvl");
     return 0;

@@ -1509,14 +1509,10 @@ int launch_pv(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
     if (p->max_ctx > PV_ATT_MAX) return nmx_attn_long(ctx, a, KVT, p->scores);
     const unsigned pgrid = (unsigned)((p->hd / PV_DS) * p->nh * p->n);
     const size_t plds = ((size_t)4 * cm_stride(p->max_ctx) + 4 + (size_t)PV_DS * PV_RS) * 4;
-    static bool pv_ready = false; /* idempotent */
-    if (!pv_ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)attn_pv_k<KVT>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)((4 * (size_t)cm_stride(PV_ATT_MAX) + 4 +
-                                                (size_t)PV_DS * PV_RS) * 4)));
-        pv_ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)attn_pv_k<KVT>,
+                    ((size_t)4 * cm_stride(PV_ATT_MAX) + 4 + (size_t)PV_DS * PV_RS) * 4, lds_set))
+        return -1;
     attn_pv_k<KVT><<<pgrid, 256, plds, ctx->stream>>>(p->scores, a.pos, a.vc, a.pos_off, a.max_ctx,
                                                        a.nh, a.nkv, a.hd, a);
     NMX_LAUNCHED(ctx, "attn_pv");
@@ -1525,7 +1521,7 @@ int launch_pv(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
 
 /* attn_qk_k + the P.V launch of launch_attn; outside attn_qk_k's limits, and for passes of
  * more than 8 tokens (prefill chunks: each of their workgroups would redo up to 32 key rows'
- * norms, measured slower than the separate launch), the three launches */
+ * norms, measured slower than the separate launch), the separate launches */
 template <int KVT>
 int launch_attn_fused(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
     if (p->hd != QK_HD || p->nh / p->nkv > 4 || p->n > QK_NMAX) {
@@ -1535,12 +1531,8 @@ int launch_attn_fused(nmx_ctx *ctx, const nmx_attn_args *p, const Attn &a) {
     }
     constexpr int CP = 32;
     const size_t lds = ((size_t)CP * (QK_HD + 4) + (8 + (size_t)QK_NMAX) * QK_HD) * 4;
-    static bool ready = false; /* idempotent */
-    if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)attn_qk_k<CP, KVT>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)attn_qk_k<CP, KVT>, lds, lds_set)) return -1;
     dim3 grid((unsigned)((p->max_ctx + CP - 1) / CP), (unsigned)p->n, (unsigned)p->nkv);
     attn_qk_k<CP, KVT><<<grid, 256, lds, ctx->stream>>>(a.q, a.pos, a.k_in, a.v_in, a.kc, a.nh, a.nkv,
                                                         a.pos_off, a.max_ctx, a, p->scores);

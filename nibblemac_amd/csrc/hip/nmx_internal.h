@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -51,6 +52,18 @@ int nmx_fail(nmx_ctx *ctx, const char *fmt, ...) __attribute__((format(printf, 2
         hipError_t e_ = hipGetLastError();                                                  \
         if (e_ != hipSuccess) return nmx_fail((ctx), "%s launch: %s", what, hipGetErrorString(e_)); \
     } while (0)
+
+/* Let a kernel of ctx's device (current on the calling thread) use `bytes` of dynamic LDS. The
+ * attribute is kept per device, so `done`, the launch site's own, has a bit for each; contexts of
+ * several threads may get here at once and set the same value. */
+static inline int nmx_dyn_lds(nmx_ctx *ctx, const void *kernel, size_t bytes,
+                              std::atomic<uint64_t> &done) {
+    const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
+    if (done.load(std::memory_order_relaxed) & bit) return 0;
+    NMX_HIP(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    done.fetch_or(bit, std::memory_order_relaxed);
+    return 0;
+}
 
 /* One matrix of a small-row Q4K matmul launch. */
 struct nmx_mt_seg {

@@ -311,12 +311,8 @@ template <int KP, int TB>
 int launch_rulec(nmx_ctx *ctx, const nmx_lin_args &a, const float *raw, int raw_stride, float *conv,
                  int C) {
     const size_t lds = (2 * (size_t)RC_TOK * rc_row(16 * KP) + 2 * RC_TOK * RC_JW + 2 * RC_TOK) * 4;
-    static bool ready = false; /* idempotent */
-    if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)lin_rulec_k<KP, TB>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)lin_rulec_k<KP, TB>, lds, lds_set)) return -1;
     const dim3 grid((unsigned)a.heads, (unsigned)(a.dv / RC_JW));
     lin_rulec_k<KP, TB><<<grid, 256, lds, ctx->stream>>>(a, raw, raw_stride, conv, C);
     NMX_LAUNCHED(ctx, "lin_rulec");

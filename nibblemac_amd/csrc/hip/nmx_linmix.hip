@@ -430,12 +430,8 @@ __global__ __launch_bounds__(MIX_MAX_THREADS) void lin_mix_k(
 
 template <int DK4>
 int launch_mix(nmx_ctx *ctx, const LinMix &m, size_t lds) {
-    static bool ready = false; /* idempotent */
-    if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)lin_mix_k<DK4>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, MIX_LDS));
-        ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)lin_mix_k<DK4>, MIX_LDS, lds_set)) return -1;
     lin_mix_k<DK4><<<dim3((unsigned)m.heads), dim3((unsigned)(4 * m.dv)), lds, ctx->stream>>>(
         m.raw, m.z, m.a_in, m.b_in, m.raw_stride, m.z_stride, m.g_stride, m.kd, m.rep, m.dv, m.n, m);
     NMX_LAUNCHED(ctx, "lin_mix");

@@ -794,12 +794,10 @@ template <int NV, bool NORM, bool SWI, int BPU, bool PAIR = false>
 int launch_one(nmx_ctx *ctx, const MtTab &tab, int groups, int cols, int n, int v0, int R, int T,
                const int8_t *q, const float *d, const float *fs, const nmx_norm_in &nm,
                nmx_a8 out, const nmx_mt_pair *pair = nullptr) {
-    static bool ready = false; /* idempotent: a racing second call sets the same value */
-    if (!ready) {
-        NMX_HIP(ctx, hipFuncSetAttribute((const void *)q4k_mt_k<NV, NORM, SWI, BPU, PAIR>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, MT_LDS));
-        ready = true;
-    }
+    static std::atomic<uint64_t> lds_set;
+    if (nmx_dyn_lds(ctx, (const void *)q4k_mt_k<NV, NORM, SWI, BPU, PAIR>,
+                    MT_LDS, lds_set))
+        return -1;
     if (const char *why = mt_geometry_error(cols, NV, R, T, BPU, NORM, SWI, PAIR))
         return nmx_fail(ctx, "q4k_mt: geometry cols=%d nv=%d R=%d T=%d bpu=%d: %s", cols, NV, R,
                         T, BPU, why);

@@ -1342,13 +1342,10 @@ int launch_mm(nmx_ctx *ctx, SegTable tab, int cols, int n, const int8_t *q, cons
         if (parts > vtiles) parts = vtiles;
         int T = (vtiles + parts - 1) / parts;
         if (T > MN_T) T = MN_T;
-        static bool ready = false; /* idempotent */
-        if (!ready) {
-            NMX_HIP(ctx, hipFuncSetAttribute((const void *)q4k_mmn_k,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             mn_lds(MN_S, MN_T, true).total));
-            ready = true;
-        }
+        static std::atomic<uint64_t> lds_set;
+        if (nmx_dyn_lds(ctx, (const void *)q4k_mmn_k,
+                        mn_lds(MN_S, MN_T, true).total, lds_set))
+            return -1;
         const dim3 grid((unsigned)groups, (unsigned)((vtiles + T - 1) / T));
         q4k_mmn_k<<<grid, 64 * S, (size_t)mn_lds(S, T, nsb > S).total, ctx->stream>>>(tab, cols, n, T, q, d, fs);
     }
